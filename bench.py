@@ -47,14 +47,11 @@ def kernel_symbol(kind, d, narrow, nt, n):
     if narrow and 2 * P <= 64:
         M, P = M // 2, 2 * P
     if kind == "grad" and d == "x":
-        st = "PassGrad<1, true, false, 0, false>"
+        st = "PassGrad<0, 1, false>"
     elif kind == "grad":
-        if nt == 256 and M == 8 and P == 32:
-            st = "PassGrad<2, true, false, 2, true>"
-        else:
-            st = "PassGrad<1, %s, false, 2, false>" % ("true" if nt == 1024 else "false")
+        st = "PassGrad<2, 2, true>" if nt == 256 and M == 8 and P == 32 else "PassGrad<2, 1, false>"
     elif kind == "grad_cross":
-        st = "PassGrad<1, true, true, 4, false>" if nt == 1024 else "PassGrad<2, false, true, 4, false>"
+        st = "PassGrad<1, 2, false>"
     elif kind == "lap_se":
         st = "PassLapSE<%s>" % ("false" if d == "x" else "true")
     else:

@@ -205,14 +205,25 @@ double kind_fields(int kind, int dir, const st::PassArgs &a)
     }
 }
 
+// The tables of direction dir in layout set lay (0: M points per lane, 3:
+// M/2) and the derivatives' right-hand-side scales.
+void set_tab(const st_ctx *c, st::PassArgs &a, int lay, int dir, double cadd)
+{
+    const st::DirTab &t = c->th[lay + dir];
+    const st::Coef &C = c->C;
+    a.tab_ = c->td + lay + dir;
+    const double k1 = cadd * c->sx1[dir] * (double)(t.n - 1) * t.op[0].scale;   // fac of src/derivCDopt6_periodic.f:181
+    const double k2 = t.s2 * t.op[1].scale;
+    a.K1 = {k1, k1 * C.a1, k1 * C.b1};
+    a.K2 = {k2, k2 * C.a2, k2 * C.b2, k2 * C.c2, k2 * C.d2};
+}
+
 int pass(st_ctx *c, int kind, int dir, st::PassArgs a, double cadd = 1.0)
 {
     const int pk = kind * 3 + dir;
     const int lay = c->force_narrow || c->cfg_narrow[kind][dir] ? 3 : 0;
     const st::DirTab &t = c->th[lay + dir];
-    a.tab = c->td + lay + dir;
-    a.K1 = cadd * c->sx1[dir] * (double)(t.n - 1) * t.op[0].scale;   // fac of src/derivCDopt6_periodic.f:181
-    a.K2 = t.s2 * t.op[1].scale;
+    set_tab(c, a, lay, dir, cadd);
     if (c->rec) {
         c->rec->push_back(Rec{kind, dir, a, &t});
         return 0;
@@ -235,9 +246,7 @@ int pass(st_ctx *c, int kind, int dir, st::PassArgs a, double cadd = 1.0)
         const int la = alt ? 3 - lay : lay;
         const st::DirTab &u = c->th[la + dir];
         st::PassArgs b = a;
-        b.tab = c->td + la + dir;
-        b.K1 = cadd * c->sx1[dir] * (double)(u.n - 1) * u.op[0].scale;
-        b.K2 = u.s2 * u.op[1].scale;
+        set_tab(c, b, la, dir, cadd);
         for (int w = alt ? 1024 : nt / 2; w >= 256 && err == hipErrorInvalidValue; w /= 2) {
             if ((w == 1024 && (u.P < 32 || (u.M & (u.M - 1)))) || lot % (w / u.P)) continue;
             err = st::run_pass(kind, u, w, dir, c->My, c->Mz, c->Mx, b, c->s);
@@ -343,7 +352,6 @@ extern "C" int st_batch_create(const st_grid *grid, const st_params *params, int
     st::Coef &C = c->C;
     C.a1 = 14.0 / 18.0;
     C.b1 = 1.0 / 36.0;
-    C.c1 = 0.0;
     C.a2 = 12.0 / 11.0;
     C.b2 = 3.0 / 44.0;
     if (params->d2_mode == 1) {
@@ -381,6 +389,12 @@ extern "C" int st_batch_create(const st_grid *grid, const st_params *params, int
             return -2;
         }
         if (!narrow) c->th[3 + d] = c->th[d];
+        for (int op = 0; op < 2; op++)      // the in-row scans rely on it
+            if (std::pow(std::fabs(c->th[d].op[op].a1), st::SCAN_REACH[op]) >= 0x1p-60) {
+                fail(c, -2, "operator %d of direction %d does not decay within %d points", op, d, st::SCAN_REACH[op]);
+                *out = c;
+                return -2;
+            }
     }
     hipError_t e;
     if ((e = hipStreamCreateWithFlags(&c->s, hipStreamNonBlocking)) != hipSuccess) {

@@ -25,6 +25,14 @@ namespace st {
 
 constexpr int HALO = 4;
 
+// The operator tables are read-only for every kernel: constant address
+// space, so that entries that are the same on every lane are scalar loads
+// also after a kernel's own global stores (a pass's second compute phase),
+// which the compiler could not prove for a plain pointer.
+#define ST_CONST __attribute__((address_space(4)))
+typedef const ST_CONST OpTab CTab;
+typedef const ST_CONST DirTab CDir;
+
 // Tile geometry of one pass launch.
 struct Geo {
     int dir;               // 0: x (stride My*Mz), 1: y (stride 1), 2: z (stride My)
@@ -182,27 +190,31 @@ DEV Lane<M, P, NP, AL> make_lane(double *lds, int ss)
     return L;
 }
 
-// Window of M own values plus HALO on each side, fetched from neighbours.
+// Window of M own values plus H on each side, fetched from neighbours (W =
+// M + 2 H; H = 4 where the operator reaches that far, 2 for the periodic
+// derivatives).
 // On a non-periodic line the points beyond either end are the mirror
 // images f(-m) = f(m), f(n-1+m) = f(n-1-m) (the symmetry of
 // src/filters_nonperiodic1d.f:830-943); the compact operators overwrite
 // their closure rows and never read them.
-template <int M, int P, bool NP, bool AL>
-DEV void window(const double (&v)[M], const Lane<M, P, NP, AL> &L, double (&w)[M + 2 * HALO])
+template <int M, int W, int P, bool NP, bool AL>
+DEV void window(const double (&v)[M], const Lane<M, P, NP, AL> &L, double (&w)[W])
 {
+    constexpr int H = (W - M) / 2;
+    static_assert(W == M + 2 * H && (!NP || H == HALO), "window width");
 #pragma unroll
-    for (int k = 0; k < M; k++) w[HALO + k] = v[k];
+    for (int k = 0; k < M; k++) w[H + k] = v[k];
 #pragma unroll
-    for (int o = 1; o <= HALO; o++) {
+    for (int o = 1; o <= H; o++) {
         const int dl = (o + M - 1) / M;
         const int idx = dl * M - o;
-        w[HALO - o] = __shfl(v[idx], L.src(-dl));
+        w[H - o] = __shfl(v[idx], L.src(-dl));
     }
 #pragma unroll
-    for (int o = 0; o < HALO; o++) {
+    for (int o = 0; o < H; o++) {
         const int dl = 1 + o / M;
         const int idx = o % M;
-        w[HALO + M + o] = __shfl(v[idx], L.src(dl));
+        w[H + M + o] = __shfl(v[idx], L.src(dl));
     }
     if constexpr (NP) {
         constexpr int n = M * P;
@@ -231,6 +243,11 @@ DEV void window(const double (&v)[M], const Lane<M, P, NP, AL> &L, double (&w)[M
     }
 }
 
+// Half-width of the window that the derivatives need on a line: +-2, and
+// the full one on a non-periodic line (the closure rows reach further).
+template <bool NP>
+constexpr int d_halo() { return NP ? HALO : 2; }
+
 // ---- cyclic solves ------------------------------------------------------
 //
 // The lane-to-lane traffic of a solve runs on DPP (data-parallel
@@ -240,7 +257,9 @@ DEV void window(const double (&v)[M], const Lane<M, P, NP, AL> &L, double (&w)[M
 constexpr int DPP_ROW_SHL = 0x100;      // + d: lane i <- lane i+d within its 16-lane row
 constexpr int DPP_ROW_SHR = 0x110;      // + d: lane i <- lane i-d within its row
 constexpr int DPP_WAVE_SHL1 = 0x130;    // lane i <- lane i+1 across the wave
+constexpr int DPP_WAVE_ROL1 = 0x134;    // the same around the wave: lane 63 <- lane 0
 constexpr int DPP_WAVE_SHR1 = 0x138;    // lane i <- lane i-1 across the wave
+constexpr int DPP_WAVE_ROR1 = 0x13c;    // the same around the wave: lane 0 <- lane 63
 constexpr int DPP_ROW_NEWBCAST = 0x150; // + k: every lane of a row <- lane k of the row
 
 // Lanes whose source lies outside the row (or the wave) read 0.
@@ -259,10 +278,19 @@ DEV double rdlane(double x)
                             __builtin_amdgcn_readlane(__double2loint(x), LANE));
 }
 
+// The same for the 16-lane rows in ROWS (bit r: row r); the others take old.
+template <int CTRL, int ROWS>
+DEV double dpp_rows(double old, double x)
+{
+    const int lo = __builtin_amdgcn_update_dpp(__double2loint(old), __double2loint(x), CTRL, ROWS, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(__double2hiint(old), __double2hiint(x), CTRL, ROWS, 0xf, false);
+    return __hiloint2double(hi, lo);
+}
+
 // y += m t for the carried state: a scalar (order 1, m[0]) or a 2-vector
 // with the row-major 2x2 matrix m (order 2).
 template <int K>
-DEV void madd(const double *m, const double (&t)[K], double (&y)[K])
+DEV void madd(const ST_CONST double *m, const double (&t)[K], double (&y)[K])
 {
     if (K == 1) {
         y[0] = fma(m[0], t[0], y[0]);
@@ -274,7 +302,7 @@ DEV void madd(const double *m, const double (&t)[K], double (&y)[K])
 }
 
 template <int K>
-DEV void madd_to(const double *m, const double (&t)[K], const double (&x)[K], double (&y)[K])
+DEV void madd_to(const ST_CONST double *m, const double (&t)[K], const double (&x)[K], double (&y)[K])
 {
 #pragma unroll
     for (int i = 0; i < K; i++) y[i] = x[i];
@@ -285,7 +313,7 @@ DEV void madd_to(const double *m, const double (&t)[K], const double (&x)[K], do
 // backward e_c += A^(M D) e_(c+D).  Rows are segment boundaries for P >= 16;
 // for P = 8 two lines share a row and the cross-line source is masked.
 template <int K, bool FWD, int D, int J, int P>
-DEV void row_step(double (&e)[K], const OpTab &T, int c)
+DEV void row_step(double (&e)[K], CTab &T, int c)
 {
     double t[K];
 #pragma unroll
@@ -309,7 +337,7 @@ DEV void sel(bool p, const double (&a)[K], const double (&b)[K], double (&y)[K])
 // On return e is the inclusive prefix (forward) or suffix (backward) state,
 // and tot the line's total (the state at its last, resp. first, lane).
 template <int K, bool FWD, int P>
-DEV void wave_scan(double (&e)[K], double (&tot)[K], const OpTab &T, int c)
+DEV void wave_scan(double (&e)[K], double (&tot)[K], CTab &T, int c)
 {
     static_assert(P == 8 || P == 16 || P == 32 || P == 64, "lanes per line");
     row_step<K, FWD, 1, 0, P>(e, T, c);
@@ -333,7 +361,7 @@ DEV void wave_scan(double (&e)[K], double (&tot)[K], const OpTab &T, int c)
         } else {
             // P = 32 or 64: carry whole rows with uniform values read from
             // one lane per row (its row-local end state), A16 = A^(16 M).
-            const double *A16 = T.sc[4];
+            const ST_CONST double *A16 = T.sc[4];
             const int row = (threadIdx.x >> 4) & 3;
             double s0[K], s1[K], s2[K], s3[K], carry[K];
 #pragma unroll
@@ -383,13 +411,74 @@ DEV void wave_scan(double (&e)[K], double (&tot)[K], const OpTab &T, int c)
     }
 }
 
-// Cyclic solve of one line per P lanes; r holds the lane's M right-hand
-// sides (the scale 1+rho^2 or 1/kappa already folded in) and returns x.
-// Order 1: x = (1 - rho S^-1)^-1 (1 - rho S)^-1 r,
-// order 2: x = (1 - a1 S^-1 - a2 S^-2)^-1 (1 - a1 S - a2 S^2)^-1 r.
-template <int K, int M, int P, bool NP, bool AL>
-DEV void solve(double (&r)[M], const OpTab &T, const Lane<M, P, NP, AL> &L)
+// The derivatives' recurrences forget quickly: their root rho (0.382 for
+// D1's alpha = 1/3, 0.188 for D2's 2/11) falls below 2^-60 within
+// SCAN_REACH points (st_create checks the tables against it).  A chunk's
+// incoming state then needs only the chunks that many points back, so the
+// scan can stop at the lane row: SCAN_STEPS doubling steps inside a 16-lane
+// row, and one carry from the end of the row before it.
+template <int OP>
+constexpr int scan_steps(int M, int P)
 {
+    constexpr int reach = SCAN_REACH[OP];
+    if (P < 16 || reach == 0) return 0;
+    for (int j = 1; j <= 4; j++)
+        if ((M << j) >= reach) return j;
+    return 0;                            // a row of 16 chunks is too short: the full scan
+}
+
+// Incoming state of each chunk from the chunk-end states e (order 1): the
+// in-row prefix (suffix) by doubling, exclusive, plus the end state of the
+// row before (after) it, times A^(M j) for the j chunks of the row in between.
+// The rows of a line follow each other around it (NP: nothing enters at
+// the first).  A wave shift by one lane hands each row's first (last) lane
+// that state and a row broadcast spreads it; for P = 64 the shift rotates,
+// for P = 32 the first (last) row of each line takes its own line's end.
+// 7 vector instructions a direction beside the doubling steps (15 for P =
+// 32), against about 45 for the full scan with its carry chain over rows,
+// cyclic total and per-lane injections.
+template <bool FWD, int STEPS, int M, int P, bool NP>
+DEV double scan_in(double e, CTab &T, int c)
+{
+    static_assert(P >= 16 && STEPS >= 1 && STEPS <= 4, "in-row scan");
+    double s[1] = {e};
+    row_step<1, FWD, 1, 0, P>(s, T, c);
+    if constexpr (STEPS >= 2) row_step<1, FWD, 2, 1, P>(s, T, c);
+    if constexpr (STEPS >= 3) row_step<1, FWD, 4, 2, P>(s, T, c);
+    if constexpr (STEPS >= 4) row_step<1, FWD, 8, 3, P>(s, T, c);
+    e = s[0];
+    const double x = FWD ? dpp<DPP_ROW_SHR + 1>(e) : dpp<DPP_ROW_SHL + 1>(e);
+    if constexpr (P == 16) {
+        if constexpr (NP) return x;
+        const double b = FWD ? dpp<DPP_ROW_NEWBCAST + 15>(e) : dpp<DPP_ROW_NEWBCAST + 0>(e);
+        return fma(T.lp[FWD ? (c & 15) : 15 - (c & 15)][0], b, x);
+    } else {
+        constexpr int SPREAD = FWD ? DPP_ROW_NEWBCAST + 0 : DPP_ROW_NEWBCAST + 15;
+        double b;
+        if constexpr (P == 64) {
+            b = NP ? dpp<SPREAD>(FWD ? dpp<DPP_WAVE_SHR1>(e) : dpp<DPP_WAVE_SHL1>(e))
+                   : dpp<SPREAD>(FWD ? dpp<DPP_WAVE_ROR1>(e) : dpp<DPP_WAVE_ROL1>(e));
+        } else {
+            double o = 0.0;                // what enters each line's first (last) row
+            if constexpr (!NP) {
+                const double s0 = rdlane<FWD ? 31 : 0>(e), s1 = rdlane<FWD ? 63 : 32>(e);
+                o = (threadIdx.x & 32) ? s1 : s0;
+            }
+            b = dpp_rows<SPREAD, FWD ? 0xa : 0x5>(o, FWD ? dpp<DPP_WAVE_SHR1>(e) : dpp<DPP_WAVE_SHL1>(e));
+        }
+        return fma(T.lp[FWD ? (c & 15) : 15 - (c & 15)][0], b, x);
+    }
+}
+
+// Cyclic solve of one line per P lanes for operator OP (0: first derivative,
+// 1: second, 2: filter); r holds the lane's M right-hand sides (the scale
+// 1+rho^2 or 1/kappa already folded in) and returns x.
+// Order 1 (OP 0, 1): x = (1 - rho S^-1)^-1 (1 - rho S)^-1 r,
+// order 2: x = (1 - a1 S^-1 - a2 S^-2)^-1 (1 - a1 S - a2 S^2)^-1 r.
+template <int OP, int M, int P, bool NP, bool AL>
+DEV void solve(double (&r)[M], CTab &T, const Lane<M, P, NP, AL> &L)
+{
+    constexpr int K = OP == 2 ? 2 : 1, STEPS = scan_steps<OP>(M, P);
     const double a1 = T.a1, a2 = T.a2;
     const int c = L.c;
     // forward recurrence inside the chunk (zero incoming state)
@@ -397,6 +486,17 @@ DEV void solve(double (&r)[M], const OpTab &T, const Lane<M, P, NP, AL> &L)
     for (int k = 1; k < M; k++) {
         r[k] = fma(a1, r[k - 1], r[k]);
         if (K == 2 && k >= 2) r[k] = fma(a2, r[k - 2], r[k]);
+    }
+    if constexpr (STEPS > 0) {
+        const double cf = scan_in<true, STEPS, M, P, NP>(r[M - 1], T, c);
+#pragma unroll
+        for (int k = 0; k < M; k++) r[k] = fma(T.cf[k][0], cf, r[k]);
+#pragma unroll
+        for (int k = M - 2; k >= 0; k--) r[k] = fma(a1, r[k + 1], r[k]);
+        const double cb = scan_in<false, STEPS, M, P, NP>(r[0], T, c);
+#pragma unroll
+        for (int k = 0; k < M; k++) r[k] = fma(T.cf[M - 1 - k][0], cb, r[k]);
+        return;
     }
     double e[K], tot[K], w[K], cin[K];
     e[0] = r[M - 1];
@@ -462,10 +562,10 @@ DEV double line_value(const double (&x)[M], const Lane<M, P, NP, AL> &L, int row
 
 // Boundary correction x -= Z q, q = G yb (the np_* tables of OpTab; Z
 // itself is applied through the recurrences, below).
-template <int MB, int M, int P, bool NP, bool AL>
-DEV void np_fix(double (&x)[M], const OpTab &T, const Lane<M, P, NP, AL> &L)
+template <int OP, int M, int P, bool NP, bool AL>
+DEV void np_fix(double (&x)[M], CTab &T, const Lane<M, P, NP, AL> &L)
 {
-    constexpr int n = M * P;
+    constexpr int n = M * P, MB = OP == 2 ? 6 : 4;
     double yb[10];
 #pragma unroll
     for (int t = 0; t < 5; t++) {
@@ -485,7 +585,7 @@ DEV void np_fix(double (&x)[M], const OpTab &T, const Lane<M, P, NP, AL> &L)
     // side that is zero away from them, instead of the MB columns of Z per
     // point (which, read once per kernel, would hold MB*M registers per
     // operator, and read at each use, wait on memory in every solve)
-    constexpr int K = MB == 6 ? 2 : 1, H = MB / 2;
+    constexpr int H = MB / 2;
     double z[M];
 #pragma unroll
     for (int k = 0; k < M; k++) {
@@ -498,7 +598,7 @@ DEV void np_fix(double (&x)[M], const OpTab &T, const Lane<M, P, NP, AL> &L)
         }
         z[k] = v;
     }
-    solve<K, M>(z, T, L);
+    solve<OP, M>(z, T, L);
 #pragma unroll
     for (int k = 0; k < M; k++) x[k] -= z[k];
 }
@@ -587,39 +687,50 @@ DEV void closure_rows(const double (&w)[M + 2 * HALO], double K, const Lane<M, P
 
 // ---- operators on a window -----------------------------------------------
 
-// First derivative: K = cadd*sx(1)*(N-1)*(1+rho^2).
-template <int M, int P, bool NP, bool AL>
-DEV void op_d1(const double (&w)[M + 2 * HALO], const Coef &C, double K, const OpTab &T,
-               const Lane<M, P, NP, AL> &L, double (&out)[M])
+// First derivative: K.k = cadd*sx(1)*(N-1)*(1+rho^2), K.a, K.b its products
+// with the stencil's weights on +-1 and +-2.
+template <int M, int W, int P, bool NP, bool AL>
+DEV void op_d1(const double (&w)[W], const Scale1 &K, CTab &T, const Lane<M, P, NP, AL> &L, double (&out)[M])
 {
+    constexpr int H = (W - M) / 2;
 #pragma unroll
     for (int k = 0; k < M; k++) {
-        const int i = k + HALO;
-        out[k] = K * ((C.c1 * (w[i + 3] - w[i - 3]) + C.b1 * (w[i + 2] - w[i - 2])) + C.a1 * (w[i + 1] - w[i - 1]));
+        const int i = k + H;
+        out[k] = fma(K.a, w[i + 1] - w[i - 1], K.b * (w[i + 2] - w[i - 2]));
     }
-    if constexpr (NP) closure_rows<0>(w, K, L, out);
-    solve<1, M>(out, T, L);
-    if constexpr (NP) np_fix<4>(out, T, L);
+    if constexpr (NP) closure_rows<0>(w, K.k, L, out);
+    solve<0, M>(out, T, L);
+    if constexpr (NP) np_fix<0>(out, T, L);
 }
 
-// Second derivative: K = (N-1)^2*sx(2)*(1+rho^2).
-template <int M, int P, bool NP, bool AL>
-DEV void op_d2(const double (&w)[M + 2 * HALO], const Coef &C, double K, const OpTab &T,
-               const Lane<M, P, NP, AL> &L, double (&out)[M])
+// Second derivative: K.k = (N-1)^2*sx(2)*(1+rho^2), K.a, K.b, K.c its products
+// with the weights on +-1, +-2 and (the coefficients as shipped only,
+// 0 otherwise) +-3, K.d with the centre weight.
+template <int M, int W, int P, bool NP, bool AL>
+DEV void op_d2(const double (&w)[W], const Scale2 &K, CTab &T, const Lane<M, P, NP, AL> &L, double (&out)[M])
 {
+    constexpr int H = (W - M) / 2;
 #pragma unroll
     for (int k = 0; k < M; k++) {
-        const int i = k + HALO;
-        out[k] = K * (((C.c2 * (w[i + 3] + w[i - 3]) + C.b2 * (w[i + 2] + w[i - 2])) + C.a2 * (w[i + 1] + w[i - 1])) - C.d2 * w[i]);
+        const int i = k + H;
+        out[k] = fma(K.a, w[i + 1] + w[i - 1], fma(K.b, w[i + 2] + w[i - 2], -K.d * w[i]));
     }
-    if constexpr (NP) closure_rows<1>(w, K, L, out);
+    if (K.c != 0.0) {                      // the same on every lane
+        double v[M], x[M + 2 * HALO];
+#pragma unroll
+        for (int k = 0; k < M; k++) v[k] = w[k + H];
+        window<M>(v, L, x);
+#pragma unroll
+        for (int k = 0; k < M; k++) out[k] = fma(K.c, x[k + HALO + 3] + x[k + HALO - 3], out[k]);
+    }
+    if constexpr (NP) closure_rows<1>(w, K.k, L, out);
     solve<1, M>(out, T, L);
-    if constexpr (NP) np_fix<4>(out, T, L);
+    if constexpr (NP) np_fix<1>(out, T, L);
 }
 
 // Eighth-order compact filter: K = 1/kappa.
 template <int M, int P, bool NP, bool AL>
-DEV void op_filt(const double (&w)[M + 2 * HALO], const Coef &C, double K, const OpTab &T,
+DEV void op_filt(const double (&w)[M + 2 * HALO], const Coef &C, double K, CTab &T,
                  const Lane<M, P, NP, AL> &L, double (&out)[M])
 {
 #pragma unroll
@@ -630,7 +741,7 @@ DEV void op_filt(const double (&w)[M + 2 * HALO], const Coef &C, double K, const
     }
     if constexpr (NP) closure_rows<2>(w, K, L, out);
     solve<2, M>(out, T, L);
-    if constexpr (NP) np_fix<6>(out, T, L);
+    if constexpr (NP) np_fix<2>(out, T, L);
 }
 
 // Truncated Gaussian (explicit).

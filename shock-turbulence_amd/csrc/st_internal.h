@@ -38,6 +38,10 @@ struct OpTab {
     double npG[6][10];
 };
 
+// Points after which operator 0 (first derivative) and 1 (second) have
+// forgotten a value: rho^reach < 2^-60.  0: no such bound is used (filter).
+constexpr int SCAN_REACH[3] = {44, 25, 0};
+
 // Per-direction operator tables and stencil factors.
 struct DirTab {
     OpTab op[3];          // 0: first derivative, 1: second derivative, 2: compact filter
@@ -50,10 +54,19 @@ struct DirTab {
 
 // Compact-scheme coefficients (src/header:191-203, src/LES_header:104-157).
 struct Coef {
-    double a1, b1, c1;            // D1 right-hand side
+    double a1, b1;                // D1 right-hand side (+-1, +-2)
     double a2, b2, c2, d2;        // D2 right-hand side (+-1, +-2, +-3, centre)
     double f0, f1, f2, f3, f4;    // compact filter right-hand side
     double g0, g1, g2, g3, g4;    // Gaussian
+};
+
+// Right-hand-side scale of the derivatives (stencil factor x solve scale)
+// and its products with the stencil's weights.
+struct Scale1 {
+    double k, a, b;               // +-1, +-2
+};
+struct Scale2 {
+    double k, a, b, c, d;         // +-1, +-2, +-3, centre
 };
 
 // Physical parameters used in kernels.

@@ -9,10 +9,11 @@ namespace st {
 
 // Everything a pass may read or write.  Unused pointers stay null.
 struct PassArgs {
-    const DirTab *tab;    // device copy of this direction's tables
+    const DirTab *tab_;   // device copy of this direction's tables (tab() in kernels)
     Coef C;
     Phys ph;
-    double K1, K2;        // D1 / D2 right-hand-side scale (stencil factor x solve scale)
+    Scale1 K1;            // D1 and D2 right-hand-side scales
+    Scale2 K2;
     long N;               // points per field
     double *Q, *QW, *dQ;  // state, RK register, right-hand side (5 fields each)
     double *G;            // 12 first derivatives, G[(3*d + i)*N] = du_i/dx_d, G[(9+d)*N] = dT/dx_d
@@ -42,6 +43,11 @@ struct PassArgs {
     const double *spg;
     int spg_left;         // x indices below this take the left state
     int pad3_;
+    // the tables, in the constant address space (no kernel writes them)
+    __device__ __forceinline__ const __attribute__((address_space(4))) DirTab *tab() const
+    {
+        return (const __attribute__((address_space(4))) DirTab *)tab_;
+    }
 };
 
 // The parameters of slot `slot` (its 1/Re and dt) over the launch-wide ones.
@@ -87,7 +93,9 @@ constexpr int RAGGED_P[4] = {16, 16, 32, 32};
 // Family member of a line length (-1: not in the family).
 int ragged_member(int n);
 hipError_t run_pass_ragged(int kind, const RaggedSpec &sp, hipStream_t s);
-hipError_t launch_grad_ragged(int kind, const RaggedSpec &sp, hipStream_t s);
+hipError_t launch_grad_x_ragged(const RaggedSpec &sp, hipStream_t s);
+hipError_t launch_grad_y_ragged(const RaggedSpec &sp, hipStream_t s);
+hipError_t launch_grad_z_ragged(const RaggedSpec &sp, hipStream_t s);
 hipError_t launch_lapse_ragged(int kind, const RaggedSpec &sp, hipStream_t s);
 hipError_t launch_hyper_ragged(int kind, const RaggedSpec &sp, hipStream_t s);
 hipError_t launch_hdivrk_ragged(int kind, const RaggedSpec &sp, hipStream_t s);
@@ -99,7 +107,9 @@ void pass_default_cfg(int kind, int dir, int *narrow, int *nt);
 hipError_t run_pass(int kind, const DirTab &t, int nt, int dir, int My, int Mz, int Mx, const PassArgs &a, hipStream_t s);
 // per translation unit (st_pass_*.hip)
 hipError_t launch_ops(int kind, const DirTab &t, int nt, int dir, int My, int Mz, int Mx, const PassArgs &a, hipStream_t s);
-hipError_t launch_grad(int kind, const DirTab &t, int nt, int dir, int My, int Mz, int Mx, const PassArgs &a, hipStream_t s);
+hipError_t launch_grad_x(const DirTab &t, int nt, int My, int Mz, int Mx, const PassArgs &a, hipStream_t s);
+hipError_t launch_grad_y(const DirTab &t, int nt, int My, int Mz, int Mx, const PassArgs &a, hipStream_t s);
+hipError_t launch_grad_z(const DirTab &t, int nt, int My, int Mz, int Mx, const PassArgs &a, hipStream_t s);
 hipError_t launch_lapse(int kind, const DirTab &t, int nt, int dir, int My, int Mz, int Mx, const PassArgs &a, hipStream_t s);
 hipError_t launch_hyper(int kind, const DirTab &t, int nt, int dir, int My, int Mz, int Mx, const PassArgs &a, hipStream_t s);
 hipError_t launch_hdivrk(int kind, const DirTab &t, int nt, int dir, int My, int Mz, int Mx, const PassArgs &a, hipStream_t s);

@@ -47,8 +47,14 @@ hipError_t run_pass(int kind, const DirTab &t, int nt, int dir, int My, int Mz, 
     switch (kind) {
     case K_D1: case K_D2: case K_FILT: case K_GAUSS:
         return launch_ops(kind, t, nt, dir, My, Mz, Mx, a, s);
-    case K_GRAD: case K_GRAD_CROSS:
-        return launch_grad(kind, t, nt, dir, My, Mz, Mx, a, s);
+    // x first (no mixed terms), z with two, y last with four and the
+    // pointwise assembly
+    case K_GRAD:
+        if (dir == 0) return launch_grad_x(t, nt, My, Mz, Mx, a, s);
+        if (dir == 2) return launch_grad_z(t, nt, My, Mz, Mx, a, s);
+        return hipErrorInvalidValue;
+    case K_GRAD_CROSS:
+        return dir == 1 ? launch_grad_y(t, nt, My, Mz, Mx, a, s) : hipErrorInvalidValue;
     case K_LAPSE:
         return launch_lapse(kind, t, nt, dir, My, Mz, Mx, a, s);
     case K_LAP2: case K_LAP2_LAST: case K_GAUSS_ETA: case K_GAUSS_ETA_LAST: case K_HDIV: case K_LAPSE_LAP2:
@@ -71,8 +77,12 @@ int ragged_member(int n)
 hipError_t run_pass_ragged(int kind, const RaggedSpec &sp, hipStream_t s)
 {
     switch (kind) {
-    case K_GRAD: case K_GRAD_CROSS:
-        return launch_grad_ragged(kind, sp, s);
+    case K_GRAD:
+        if (sp.dir == 0) return launch_grad_x_ragged(sp, s);
+        if (sp.dir == 2) return launch_grad_z_ragged(sp, s);
+        return hipErrorInvalidValue;
+    case K_GRAD_CROSS:
+        return sp.dir == 1 ? launch_grad_y_ragged(sp, s) : hipErrorInvalidValue;
     case K_LAPSE:
         return launch_lapse_ragged(kind, sp, s);
     case K_LAP2: case K_LAP2_LAST: case K_GAUSS_ETA: case K_GAUSS_ETA_LAST: case K_HDIV: case K_LAPSE_LAP2:

@@ -8,7 +8,9 @@
 //           Elementary Functions", 1980), |r| <= 0.347, Taylor series to r^13.
 // Series truncation is below 2^-56 relative in both; the result is within a
 // few units in the last place of the correctly rounded power.  Arguments
-// that are not positive and finite go to the library pow.
+// that are not positive and finite take pow's special values (pow_edge); the
+// library pow itself, inlined once per point, made up a third of the code of
+// the first-derivative passes, which then overflowed the instruction cache.
 //
 // Plain C++ apart from the qualifier, so that host code (and the tests) can
 // compile exactly the device arithmetic.
@@ -73,11 +75,26 @@ ST_HD double series_exp(double y)
     return std::ldexp(p, int(k));
 }
 
-// x^a for x > 0 and |a log x| < 700.
+// x^a for x that is zero, negative, infinite or NaN, as pow has it; r is
+// |x|^a for finite x != 0.
+ST_HD double pow_edge(double x, double a, double r)
+{
+    if (a == 0.0) return 1.0;
+    if (x != x) return x;
+    const double ax = std::fabs(x);
+    if (ax == 0.0) r = a > 0.0 ? 0.0 : HUGE_VAL;
+    if (ax == HUGE_VAL) r = a > 0.0 ? HUGE_VAL : 0.0;
+    if (!std::signbit(x)) return r;
+    const bool whole = std::rint(a) == a, odd = whole && std::rint(0.5 * a) != 0.5 * a;
+    if (odd) return -r;
+    return whole || ax == 0.0 || ax == HUGE_VAL ? r : NAN;
+}
+
 ST_HD double series_pow(double x, double a)
 {
-    if (!(x > 0.0) || !(x < 1.0e300)) return std::pow(x, a);
-    return series_exp(a * series_log(x));
+    double r = series_exp(a * series_log(std::fabs(x)));
+    if (!(x > 0.0 && x < HUGE_VAL)) r = pow_edge(x, a, r);
+    return r;
 }
 
 }  // namespace st

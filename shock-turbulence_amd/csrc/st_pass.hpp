@@ -12,6 +12,53 @@
 namespace st {
 
 // ---------------------------------------------------------------------
+// field access of a pass
+// ---------------------------------------------------------------------
+// NT: streaming (non-temporal) loads and stores.
+template <bool NT>
+struct GRef {
+    double *p;
+    DEV operator double() const { return NT ? __builtin_nontemporal_load(p) : *p; }
+    DEV void operator=(double v) const
+    {
+        if constexpr (NT) __builtin_nontemporal_store(v, p);
+        else *p = v;
+    }
+};
+template <bool NT>
+struct GPtr {
+    double *p;
+    DEV GRef<NT> operator[](long i) const { return {p + i}; }
+    DEV explicit operator bool() const { return p != nullptr; }
+};
+
+// The arguments as a pass sees them: every field through GPtr.
+template <bool NT>
+struct Args : PassArgs {
+    GPtr<NT> Q, QW, dQ, G, L2e, S, Cb, L2S, L4e, L4S, eta, Hc, dQp, L2ep, in0, out0, out1;
+    DEV Args(const PassArgs &b) : PassArgs(b)
+    {
+        Q = {b.Q};
+        QW = {b.QW};
+        dQ = {b.dQ};
+        G = {b.G};
+        L2e = {b.L2e};
+        S = {b.S};
+        Cb = {b.Cb};
+        L2S = {b.L2S};
+        L4e = {b.L4e};
+        L4S = {b.L4S};
+        eta = {b.eta};
+        Hc = {b.Hc};
+        dQp = {const_cast<double *>(b.dQp)};
+        L2ep = {const_cast<double *>(b.L2ep)};
+        in0 = {const_cast<double *>(b.in0)};
+        out0 = {b.out0};
+        out1 = {b.out1};
+    }
+};
+
+// ---------------------------------------------------------------------
 // generic pass kernel
 // ---------------------------------------------------------------------
 template <class PASS>
@@ -124,8 +171,9 @@ DEV void pass_body(const Geo &g, const PassArgs &a0, long tile)
     const int si = (int)(tile / g.tpi);
     const int slot = a0.slots ? a0.slots[si] : si;
     if (a0.act && !a0.act[slot]) return;          // uniform per workgroup, before any barrier
-    PassArgs a;
-    slot_params(a0, slot, a);
+    PassArgs ap;
+    slot_params(a0, slot, ap);
+    const Args<false> a(ap);
     const Walk<M, P, NT> W(g, tile - (long)si * g.tpi, (long)slot * a.ni, threadIdx.x);
     constexpr int ss = NT * M;           // slot size: B*M*P with B*P = NT
 
@@ -288,14 +336,17 @@ struct NoReuse {
     static constexpr int MIN_WAVES = 1;
     static constexpr int LOAD_UNROLL = 8;
     static constexpr int NPF = 0;
-    DEV static void prefetch(const Geo &, const PassArgs &, long, double *) {}
-    DEV static void store_early(const Geo &, const PassArgs &, long, const double *) {}
+    template <class A>
+    DEV static void prefetch(const Geo &, const A &, long, double *) {}
+    template <class A>
+    DEV static void store_early(const Geo &, const A &, long, const double *) {}
 };
 
 // ---------------------------------------------------------------------
 // helpers
 // ---------------------------------------------------------------------
-DEV double qf(const PassArgs &a, int comp, long gi) { return a.Q[comp * a.N + gi]; }
+template <class A>
+DEV double qf(const A &a, int comp, long gi) { return a.Q[comp * a.N + gi]; }
 
 template <int M, int P, bool NP, bool AL>
 DEV void qown(const Lane<M, P, NP, AL> &L, int k, double &q1, double &q2, double &q3, double &q4, double &q5)
@@ -307,9 +358,10 @@ DEV void qown(const Lane<M, P, NP, AL> &L, int k, double &q1, double &q2, double
     q5 = L.ld(4, k);
 }
 
-DEV void upd(double *p, double v, bool first)
+template <bool NT>
+DEV void upd(GRef<NT> p, double v, bool first)
 {
-    *p = first ? v : *p + v;
+    p = first ? v : p + v;
 }
 
 

@@ -18,8 +18,10 @@ struct PassFilterQ {
     // the RK update loads 15 fields per point: two points in flight at once
     static constexpr int LOAD_UNROLL = KIND == 0 ? 1 : 8;
     static constexpr int NPF = 0;
-    DEV static void prefetch(const Geo &, const PassArgs &, long, double *) {}
-    DEV static void load(const Geo &, const PassArgs &a, long gi, double (&v)[5])
+    template <class A>
+    DEV static void prefetch(const Geo &, const A &, long, double *) {}
+    template <class A>
+    DEV static void load(const Geo &, const A &a, long gi, double (&v)[5])
     {
 #pragma unroll
         for (int c = 0; c < 5; c++) {
@@ -29,18 +31,18 @@ struct PassFilterQ {
                 // update (PassHdivRkf) rounds alike; the first stage of a
                 // loop (alpha = 0) does not read QW, so the loop needs no
                 // clearing of it
-                const double qw = a.rk_a == 0.0 ? fma(a.dt, a.dQ[o], 0.0) : fma(a.dt, a.dQ[o], a.rk_a * a.QW[o]);
+                const double qw = a.rk_a == 0.0 ? fma(a.dt, (double)a.dQ[o], 0.0) : fma(a.dt, (double)a.dQ[o], a.rk_a * a.QW[o]);
                 a.QW[o] = qw;
-                v[c] = fma(a.rk_b, qw, a.Q[o]);
+                v[c] = fma(a.rk_b, qw, (double)a.Q[o]);
             } else {
                 v[c] = a.Q[o];
             }
         }
     }
-    template <int M, int P, bool NP, bool AL>
-    DEV static void compute(const Geo &, const PassArgs &a, const Lane<M, P, NP, AL> &L, double (&)[1][M])
+    template <int M, int P, bool NP, bool AL, class A>
+    DEV static void compute(const Geo &, const A &a, const Lane<M, P, NP, AL> &L, double (&)[1][M])
     {
-        const OpTab &T = a.tab->op[2];
+        CTab &T = a.tab()->op[2];
 #pragma unroll 1
         for (int m = 0; m < 5; m++) {
             double f[M], w[M + 2 * HALO], r[M];
@@ -52,8 +54,10 @@ struct PassFilterQ {
             for (int k = 0; k < M; k++) L.st(m, k, r[k]);
         }
     }
-    DEV static void store(const Geo &, const PassArgs &, long, const double *) {}
-    DEV static void store_early(const Geo &, const PassArgs &a, long gi, const double *v)
+    template <class A>
+    DEV static void store(const Geo &, const A &, long, const double *) {}
+    template <class A>
+    DEV static void store_early(const Geo &, const A &a, long gi, const double *v)
     {
         const long N = a.N;
         if (KIND == 2 && a.fix) {

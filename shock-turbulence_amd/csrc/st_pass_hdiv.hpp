@@ -20,14 +20,16 @@ struct PassHyperDiv {
     static constexpr int MIN_WAVES = 1;
     static constexpr int LOAD_UNROLL = 8;
     static constexpr int NPF = 4;            // dQ 1, 2, 3, 5 before this pass
-    DEV static void prefetch(const Geo &, const PassArgs &a, long gi, double *p)
+    template <class A>
+    DEV static void prefetch(const Geo &, const A &a, long gi, double *p)
     {
         p[0] = a.dQ[gi];
         p[1] = a.dQ[a.N + gi];
         p[2] = a.dQ[2 * a.N + gi];
         p[3] = a.dQ[4 * a.N + gi];
     }
-    DEV static void load(const Geo &g, const PassArgs &a, long gi, double (&v)[4])
+    template <class A>
+    DEV static void load(const Geo &g, const A &a, long gi, double (&v)[4])
     {
         const long N = a.N;
         fluxes(g, a, gi, a.Hc[gi], a.Hc[N + gi], a.Hc[2 * N + gi], v);
@@ -37,12 +39,12 @@ struct PassHyperDiv {
     // loads of a point issue together, which the load phases of hyper_div
     // and hdiv_rkf gain from (2-3%); the z pass of gauss_hdiv computes them
     // in its mid phase, where the branch on the direction measured faster)
-    template <bool SEL = true>
-    DEV static void fluxes(const Geo &g, const PassArgs &a, long gi, double beta, double mu, double kap,
+    template <bool SEL = true, class A>
+    DEV static void fluxes(const Geo &g, const A &a, long gi, double beta, double mu, double kap,
                            double (&v)[4])
     {
         const long N = a.N;
-        const double *G = a.G;
+        const auto G = a.G;
         const double gxx = G[gi], gyy = G[4 * N + gi], gzz = G[8 * N + gi];
         const double dil = gxx + gyy + gzz;
         const double q4 = a.Q[3 * N + gi];
@@ -82,22 +84,24 @@ struct PassHyperDiv {
         v[2] = tz;
         v[3] = uh * tx + vh * ty + wh * tz + kap * G[(9 + g.dir) * N + gi];
     }
-    template <int M, int P, bool NP, bool AL>
-    DEV static void compute(const Geo &, const PassArgs &a, const Lane<M, P, NP, AL> &L, double (&)[1][M])
+    template <int M, int P, bool NP, bool AL, class A>
+    DEV static void compute(const Geo &, const A &a, const Lane<M, P, NP, AL> &L, double (&)[1][M])
     {
 #pragma unroll 1
         for (int m = 0; m < 4; m++) {
-            double f[M], w[M + 2 * HALO], r[M];
+            double f[M], w[M + 2 * d_halo<NP>()], r[M];
 #pragma unroll
             for (int k = 0; k < M; k++) f[k] = L.ld(m, k);
             window<M>(f, L, w);
-            op_d1<M>(w, a.C, a.K1, a.tab->op[0], L, r);
+            op_d1<M>(w, a.K1, a.tab()->op[0], L, r);
 #pragma unroll
             for (int k = 0; k < M; k++) L.st(m, k, r[k]);
         }
     }
-    DEV static void store(const Geo &, const PassArgs &, long, const double *) {}
-    DEV static void store_early(const Geo &, const PassArgs &a, long gi, const double *v)
+    template <class A>
+    DEV static void store(const Geo &, const A &, long, const double *) {}
+    template <class A>
+    DEV static void store_early(const Geo &, const A &a, long gi, const double *v)
     {
         a.dQ[gi] = v[4] + v[0];
         a.dQ[a.N + gi] = v[5] + v[1];

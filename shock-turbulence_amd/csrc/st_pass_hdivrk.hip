@@ -30,8 +30,10 @@ struct PassHdivRkf {
     // the momenta and density that the fluxes read go on to the update in
     // registers (mid reads only the energy of Q)
     static constexpr int NLCARRY = 4;
-    DEV static void prefetch(const Geo &, const PassArgs &, long, double *) {}
-    DEV static void load(const Geo &g, const PassArgs &a, long gi, double (&v)[5 + NLCARRY])
+    template <class A>
+    DEV static void prefetch(const Geo &, const A &, long, double *) {}
+    template <class A>
+    DEV static void load(const Geo &g, const A &a, long gi, double (&v)[5 + NLCARRY])
     {
         double t[4];
         PassHyperDiv::load(g, a, gi, t);
@@ -41,12 +43,13 @@ struct PassHdivRkf {
 #pragma unroll
         for (int c = 0; c < 4; c++) v[5 + c] = a.Q[c * a.N + gi];
     }
-    template <int M, int P, bool NP, bool AL>
-    DEV static void compute(const Geo &g, const PassArgs &a, const Lane<M, P, NP, AL> &L, double (&o)[1][M])
+    template <int M, int P, bool NP, bool AL, class A>
+    DEV static void compute(const Geo &g, const A &a, const Lane<M, P, NP, AL> &L, double (&o)[1][M])
     {
         PassHyperDiv::compute<M, P, NP>(g, a, L, o);
     }
-    DEV static void mid(const Geo &g, const PassArgs &a, long gi, int ix, double (&v)[5], const double *lq)
+    template <class A>
+    DEV static void mid(const Geo &g, const A &a, long gi, int ix, double (&v)[5], const double *lq)
     {
         const long N = a.N;
         double dq[5];
@@ -63,7 +66,7 @@ struct PassHdivRkf {
 #pragma unroll
         for (int c = 0; c < 5; c++) {
             const long o = c * N + gi;
-            const double q = c < 4 ? lq[c] : a.Q[o];
+            const double q = c < 4 ? lq[c] : (double)a.Q[o];
             if (sg != 0.0) dq[c] = fma(-sg, q - ref[c], dq[c]);
             // as PassFilterQ<0> (alpha = 0: QW not read)
             const double qw = a.rk_a == 0.0 ? fma(a.dt, dq[c], 0.0) : fma(a.dt, dq[c], a.rk_a * a.QW[o]);
@@ -71,10 +74,10 @@ struct PassHdivRkf {
             v[c] = fma(a.rk_b, qw, q);
         }
     }
-    template <int M, int P, bool NP, bool AL>
-    DEV static void compute2(const Geo &, const PassArgs &a, const Lane<M, P, NP, AL> &L)
+    template <int M, int P, bool NP, bool AL, class A>
+    DEV static void compute2(const Geo &, const A &a, const Lane<M, P, NP, AL> &L)
     {
-        const OpTab &T = a.tab->op[2];
+        CTab &T = a.tab()->op[2];
 #pragma unroll 1
         for (int m = 0; m < 5; m++) {
             double f[M], w[M + 2 * HALO], r[M];
@@ -86,8 +89,10 @@ struct PassHdivRkf {
             for (int k = 0; k < M; k++) L.st(m, k, r[k]);
         }
     }
-    DEV static void store(const Geo &, const PassArgs &, long, const double *) {}
-    DEV static void store_early(const Geo &, const PassArgs &a, long gi, const double *v)
+    template <class A>
+    DEV static void store(const Geo &, const A &, long, const double *) {}
+    template <class A>
+    DEV static void store_early(const Geo &, const A &a, long gi, const double *v)
     {
 #pragma unroll
         for (int c = 0; c < 5; c++) a.Q[c * a.N + gi] = v[c];

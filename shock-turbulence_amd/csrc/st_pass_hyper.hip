@@ -9,28 +9,30 @@ namespace st {
 // ---------------------------------------------------------------------
 struct PassLap2 : NoReuse {
     static constexpr int NSLOT = 1, NOUT = 1, NEARLY = 0;
-    DEV static void load(const Geo &, const PassArgs &a, long gi, double (&v)[1]) { v[0] = a.L2S[gi]; }
-    template <int M, int P, bool NP, bool AL>
-    DEV static void compute(const Geo &, const PassArgs &a, const Lane<M, P, NP, AL> &L, double (&out)[1][M])
+    template <class A>
+    DEV static void load(const Geo &, const A &a, long gi, double (&v)[1]) { v[0] = a.L2S[gi]; }
+    template <int M, int P, bool NP, bool AL, class A>
+    DEV static void compute(const Geo &, const A &a, const Lane<M, P, NP, AL> &L, double (&out)[1][M])
     {
-        double f[M], w[M + 2 * HALO];
+        double f[M], w[M + 2 * d_halo<NP>()];
 #pragma unroll
         for (int k = 0; k < M; k++) f[k] = L.ld(0, k);
         window<M>(f, L, w);
-        op_d2<M>(w, a.C, a.K2, a.tab->op[1], L, out[0]);
+        op_d2<M>(w, a.K2, a.tab()->op[1], L, out[0]);
     }
-    DEV static void store(const Geo &, const PassArgs &a, long gi, const double *v) { upd(&a.L4S[gi], v[0], a.first); }
+    template <class A>
+    DEV static void store(const Geo &, const A &a, long gi, const double *v) { upd(a.L4S[gi], v[0], a.first); }
 };
 
 // D2 along the sweep of the first staged slot, in place.
-template <int M, int P, bool NP, bool AL>
-DEV void d2_slot(const PassArgs &a, const Lane<M, P, NP, AL> &L, int m)
+template <int M, int P, bool NP, bool AL, class A>
+DEV void d2_slot(const A &a, const Lane<M, P, NP, AL> &L, int m)
 {
-    double f[M], w[M + 2 * HALO], r[M];
+    double f[M], w[M + 2 * d_halo<NP>()], r[M];
 #pragma unroll
     for (int k = 0; k < M; k++) f[k] = L.ld(m, k);
     window<M>(f, L, w);
-    op_d2<M>(w, a.C, a.K2, a.tab->op[1], L, r);
+    op_d2<M>(w, a.K2, a.tab()->op[1], L, r);
 #pragma unroll
     for (int k = 0; k < M; k++) L.st(m, k, r[k]);
 }
@@ -51,19 +53,22 @@ struct PassLapSELap2 {
     static constexpr int MIN_WAVES = 1;
     static constexpr int LOAD_UNROLL = 8;
     static constexpr int NPF = 0;
-    DEV static void prefetch(const Geo &, const PassArgs &, long, double *) {}
-    DEV static void load(const Geo &, const PassArgs &a, long gi, double (&v)[2])
+    template <class A>
+    DEV static void prefetch(const Geo &, const A &, long, double *) {}
+    template <class A>
+    DEV static void load(const Geo &, const A &a, long gi, double (&v)[2])
     {
         v[0] = a.S[gi];
         v[1] = a.L2e[gi];
     }
-    template <int M, int P, bool NP, bool AL>
-    DEV static void compute(const Geo &, const PassArgs &a, const Lane<M, P, NP, AL> &L, double (&)[1][M])
+    template <int M, int P, bool NP, bool AL, class A>
+    DEV static void compute(const Geo &, const A &a, const Lane<M, P, NP, AL> &L, double (&)[1][M])
     {
 #pragma unroll 1
         for (int m = 0; m < 2; m++) d2_slot<M, P, NP>(a, L, m);
     }
-    DEV static void mid(const Geo &, const PassArgs &a, long gi, int, double (&v)[2])
+    template <class A>
+    DEV static void mid(const Geo &, const A &a, long gi, int, double (&v)[2])
     {
         const double l2s = a.L2S[gi] + v[0];       // as the accumulating D2 pass of |S| and Lap e
         a.L2S[gi] = l2s;
@@ -71,13 +76,15 @@ struct PassLapSELap2 {
         v[0] = l2s;
         v[1] = 0.0;
     }
-    template <int M, int P, bool NP, bool AL>
-    DEV static void compute2(const Geo &, const PassArgs &a, const Lane<M, P, NP, AL> &L)
+    template <int M, int P, bool NP, bool AL, class A>
+    DEV static void compute2(const Geo &, const A &a, const Lane<M, P, NP, AL> &L)
     {
         d2_slot<M, P, NP>(a, L, 0);
     }
-    DEV static void store(const Geo &, const PassArgs &, long, const double *) {}
-    DEV static void store_early(const Geo &, const PassArgs &a, long gi, const double *v) { a.L4S[gi] = v[0]; }
+    template <class A>
+    DEV static void store(const Geo &, const A &, long, const double *) {}
+    template <class A>
+    DEV static void store_early(const Geo &, const A &a, long gi, const double *v) { a.L4S[gi] = v[0]; }
 };
 
 // ---------------------------------------------------------------------
@@ -96,18 +103,21 @@ struct PassLap2Gauss {
     static constexpr int MIN_WAVES = 1;
     static constexpr int LOAD_UNROLL = 8;
     static constexpr int NPF = 0;
-    DEV static void prefetch(const Geo &, const PassArgs &, long, double *) {}
-    DEV static void load(const Geo &, const PassArgs &a, long gi, double (&v)[2])
+    template <class A>
+    DEV static void prefetch(const Geo &, const A &, long, double *) {}
+    template <class A>
+    DEV static void load(const Geo &, const A &a, long gi, double (&v)[2])
     {
         v[0] = a.L2S[gi];
         v[1] = 0.0;
     }
-    template <int M, int P, bool NP, bool AL>
-    DEV static void compute(const Geo &, const PassArgs &a, const Lane<M, P, NP, AL> &L, double (&)[1][M])
+    template <int M, int P, bool NP, bool AL, class A>
+    DEV static void compute(const Geo &, const A &a, const Lane<M, P, NP, AL> &L, double (&)[1][M])
     {
         d2_slot<M, P, NP>(a, L, 0);
     }
-    DEV static void mid(const Geo &, const PassArgs &a, long gi, int, double (&v)[2])
+    template <class A>
+    DEV static void mid(const Geo &, const A &a, long gi, int, double (&v)[2])
     {
         const Phys &ph = a.ph;
         const double d4S = fabs(a.L4S[gi] + v[0]);
@@ -118,8 +128,8 @@ struct PassLap2Gauss {
         v[0] = q4 * d4S;
         v[1] = fac3 * d4e;
     }
-    template <int M, int P, bool NP, bool AL>
-    DEV static void compute2(const Geo &, const PassArgs &a, const Lane<M, P, NP, AL> &L)
+    template <int M, int P, bool NP, bool AL, class A>
+    DEV static void compute2(const Geo &, const A &a, const Lane<M, P, NP, AL> &L)
     {
 #pragma unroll 1
         for (int m = 0; m < 2; m++) {
@@ -132,8 +142,10 @@ struct PassLap2Gauss {
             for (int k = 0; k < M; k++) L.st(m, k, r[k]);
         }
     }
-    DEV static void store(const Geo &, const PassArgs &, long, const double *) {}
-    DEV static void store_early(const Geo &, const PassArgs &a, long gi, const double *v)
+    template <class A>
+    DEV static void store(const Geo &, const A &, long, const double *) {}
+    template <class A>
+    DEV static void store_early(const Geo &, const A &a, long gi, const double *v)
     {
         a.eta[gi] = v[0];
         a.eta[a.N + gi] = v[1];
@@ -146,13 +158,14 @@ struct PassLap2Gauss {
 // ---------------------------------------------------------------------
 struct PassGaussEta : NoReuse {
     static constexpr int NSLOT = 2, NOUT = 2, NEARLY = 0;
-    DEV static void load(const Geo &, const PassArgs &a, long gi, double (&v)[2])
+    template <class A>
+    DEV static void load(const Geo &, const A &a, long gi, double (&v)[2])
     {
         v[0] = a.eta[gi];
         v[1] = a.eta[a.N + gi];
     }
-    template <int M, int P, bool NP, bool AL>
-    DEV static void compute(const Geo &, const PassArgs &a, const Lane<M, P, NP, AL> &L, double (&out)[2][M])
+    template <int M, int P, bool NP, bool AL, class A>
+    DEV static void compute(const Geo &, const A &a, const Lane<M, P, NP, AL> &L, double (&out)[2][M])
     {
 #pragma unroll
         for (int m = 0; m < 2; m++) {
@@ -163,7 +176,8 @@ struct PassGaussEta : NoReuse {
             op_gauss<M>(w, a.C, out[m]);
         }
     }
-    DEV static void store(const Geo &, const PassArgs &a, long gi, const double *v)
+    template <class A>
+    DEV static void store(const Geo &, const A &a, long gi, const double *v)
     {
         a.eta[gi] = v[0];
         a.eta[a.N + gi] = v[1];
@@ -187,16 +201,18 @@ struct PassGaussHdiv {
     static constexpr int MIN_WAVES = 1;
     static constexpr int LOAD_UNROLL = 8;
     static constexpr int NPF = PassHyperDiv::NPF;
-    DEV static void prefetch(const Geo &g, const PassArgs &a, long gi, double *p) { PassHyperDiv::prefetch(g, a, gi, p); }
-    DEV static void load(const Geo &, const PassArgs &a, long gi, double (&v)[4])
+    template <class A>
+    DEV static void prefetch(const Geo &g, const A &a, long gi, double *p) { PassHyperDiv::prefetch(g, a, gi, p); }
+    template <class A>
+    DEV static void load(const Geo &, const A &a, long gi, double (&v)[4])
     {
         v[0] = a.eta[gi];
         v[1] = a.eta[a.N + gi];
         v[2] = 0.0;
         v[3] = 0.0;
     }
-    template <int M, int P, bool NP, bool AL>
-    DEV static void compute(const Geo &, const PassArgs &a, const Lane<M, P, NP, AL> &L, double (&)[1][M])
+    template <int M, int P, bool NP, bool AL, class A>
+    DEV static void compute(const Geo &, const A &a, const Lane<M, P, NP, AL> &L, double (&)[1][M])
     {
 #pragma unroll
         for (int m = 0; m < 2; m++) {
@@ -209,7 +225,8 @@ struct PassGaussHdiv {
             for (int k = 0; k < M; k++) L.st(m, k, r[k]);
         }
     }
-    DEV static void mid(const Geo &g, const PassArgs &a, long gi, int, double (&v)[4])
+    template <class A>
+    DEV static void mid(const Geo &g, const A &a, long gi, int, double (&v)[4])
     {
         const Phys &ph = a.ph;
         const long N = a.N;
@@ -222,14 +239,16 @@ struct PassGaussHdiv {
         a.Hc[2 * N + gi] = kap;
         PassHyperDiv::fluxes<false>(g, a, gi, beta, mu, kap, v);
     }
-    template <int M, int P, bool NP, bool AL>
-    DEV static void compute2(const Geo &g, const PassArgs &a, const Lane<M, P, NP, AL> &L)
+    template <int M, int P, bool NP, bool AL, class A>
+    DEV static void compute2(const Geo &g, const A &a, const Lane<M, P, NP, AL> &L)
     {
         double o[1][M];
         PassHyperDiv::compute<M, P, NP>(g, a, L, o);
     }
-    DEV static void store(const Geo &, const PassArgs &, long, const double *) {}
-    DEV static void store_early(const Geo &g, const PassArgs &a, long gi, const double *v)
+    template <class A>
+    DEV static void store(const Geo &, const A &, long, const double *) {}
+    template <class A>
+    DEV static void store_early(const Geo &g, const A &a, long gi, const double *v)
     {
         PassHyperDiv::store_early(g, a, gi, v);
     }

@@ -18,34 +18,38 @@ struct PassLapSE {
     static constexpr int MIN_WAVES = 1;
     static constexpr int LOAD_UNROLL = 8;
     static constexpr int NPF = ACC ? 2 : 0;
-    DEV static void prefetch(const Geo &, const PassArgs &a, long gi, double *p)
+    template <class A>
+    DEV static void prefetch(const Geo &, const A &a, long gi, double *p)
     {
         if (ACC) {
             p[0] = a.L2S[gi];
             p[1] = a.L4e[gi];
         }
     }
-    DEV static void load(const Geo &, const PassArgs &a, long gi, double (&v)[2])
+    template <class A>
+    DEV static void load(const Geo &, const A &a, long gi, double (&v)[2])
     {
         v[0] = a.S[gi];
         v[1] = a.L2e[gi];
     }
-    template <int M, int P, bool NP, bool AL>
-    DEV static void compute(const Geo &, const PassArgs &a, const Lane<M, P, NP, AL> &L, double (&)[1][M])
+    template <int M, int P, bool NP, bool AL, class A>
+    DEV static void compute(const Geo &, const A &a, const Lane<M, P, NP, AL> &L, double (&)[1][M])
     {
 #pragma unroll 1
         for (int m = 0; m < 2; m++) {
-            double f[M], w[M + 2 * HALO], r[M];
+            double f[M], w[M + 2 * d_halo<NP>()], r[M];
 #pragma unroll
             for (int k = 0; k < M; k++) f[k] = L.ld(m, k);
             window<M>(f, L, w);
-            op_d2<M>(w, a.C, a.K2, a.tab->op[1], L, r);
+            op_d2<M>(w, a.K2, a.tab()->op[1], L, r);
 #pragma unroll
             for (int k = 0; k < M; k++) L.st(m, k, r[k]);
         }
     }
-    DEV static void store(const Geo &, const PassArgs &, long, const double *) {}
-    DEV static void store_early(const Geo &, const PassArgs &a, long gi, const double *v)
+    template <class A>
+    DEV static void store(const Geo &, const A &, long, const double *) {}
+    template <class A>
+    DEV static void store_early(const Geo &, const A &a, long gi, const double *v)
     {
         if constexpr (ACC) {
             a.L2S[gi] = v[2] + v[0];

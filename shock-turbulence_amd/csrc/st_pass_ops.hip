@@ -9,17 +9,19 @@ namespace st {
 // ---------------------------------------------------------------------
 struct PassD1 : NoReuse {
     static constexpr int NSLOT = 1, NOUT = 1, NEARLY = 0;
-    DEV static void load(const Geo &, const PassArgs &a, long gi, double (&v)[1]) { v[0] = a.in0[gi]; }
-    template <int M, int P, bool NP, bool AL>
-    DEV static void compute(const Geo &, const PassArgs &a, const Lane<M, P, NP, AL> &L, double (&out)[1][M])
+    template <class A>
+    DEV static void load(const Geo &, const A &a, long gi, double (&v)[1]) { v[0] = a.in0[gi]; }
+    template <int M, int P, bool NP, bool AL, class A>
+    DEV static void compute(const Geo &, const A &a, const Lane<M, P, NP, AL> &L, double (&out)[1][M])
     {
-        double f[M], w[M + 2 * HALO];
+        double f[M], w[M + 2 * d_halo<NP>()];
 #pragma unroll
         for (int k = 0; k < M; k++) f[k] = L.ld(0, k);
         window<M>(f, L, w);
-        op_d1<M>(w, a.C, a.K1, a.tab->op[0], L, out[0]);
+        op_d1<M>(w, a.K1, a.tab()->op[0], L, out[0]);
     }
-    DEV static void store(const Geo &, const PassArgs &a, long gi, const double *v)
+    template <class A>
+    DEV static void store(const Geo &, const A &a, long gi, const double *v)
     {
         a.out0[gi] = a.iadd ? a.out0[gi] + v[0] : v[0];
     }
@@ -27,24 +29,26 @@ struct PassD1 : NoReuse {
 
 struct PassD2 : NoReuse {
     static constexpr int NSLOT = 1, NOUT = 1, NEARLY = 1;
-    DEV static void load(const Geo &, const PassArgs &a, long gi, double (&v)[1]) { v[0] = a.in0[gi]; }
-    template <int M, int P, bool NP, bool AL>
-    DEV static void compute(const Geo &, const PassArgs &a, const Lane<M, P, NP, AL> &L, double (&out)[1][M])
+    template <class A>
+    DEV static void load(const Geo &, const A &a, long gi, double (&v)[1]) { v[0] = a.in0[gi]; }
+    template <int M, int P, bool NP, bool AL, class A>
+    DEV static void compute(const Geo &, const A &a, const Lane<M, P, NP, AL> &L, double (&out)[1][M])
     {
-        double f[M], w[M + 2 * HALO], d2[M];
+        double f[M], w[M + 2 * d_halo<NP>()], d2[M];
 #pragma unroll
         for (int k = 0; k < M; k++) f[k] = L.ld(0, k);
         window<M>(f, L, w);
-        op_d2<M>(w, a.C, a.K2, a.tab->op[1], L, d2);
+        op_d2<M>(w, a.K2, a.tab()->op[1], L, d2);
 #pragma unroll
         for (int k = 0; k < M; k++) L.st(1, k, d2[k]);
-        if (a.iadd) op_d1<M>(w, a.C, a.K1, a.tab->op[0], L, out[0]);
+        if (a.iadd) op_d1<M>(w, a.K1, a.tab()->op[0], L, out[0]);
         else {
 #pragma unroll
             for (int k = 0; k < M; k++) out[0][k] = 0.0;
         }
     }
-    DEV static void store(const Geo &, const PassArgs &a, long gi, const double *v)
+    template <class A>
+    DEV static void store(const Geo &, const A &a, long gi, const double *v)
     {
         if (a.iadd) a.out0[gi] = v[0];
         a.out1[gi] = v[1];
@@ -53,24 +57,27 @@ struct PassD2 : NoReuse {
 
 struct PassFilt : NoReuse {
     static constexpr int NSLOT = 1, NOUT = 1, NEARLY = 0;
-    DEV static void load(const Geo &, const PassArgs &a, long gi, double (&v)[1]) { v[0] = a.in0[gi]; }
-    template <int M, int P, bool NP, bool AL>
-    DEV static void compute(const Geo &, const PassArgs &a, const Lane<M, P, NP, AL> &L, double (&out)[1][M])
+    template <class A>
+    DEV static void load(const Geo &, const A &a, long gi, double (&v)[1]) { v[0] = a.in0[gi]; }
+    template <int M, int P, bool NP, bool AL, class A>
+    DEV static void compute(const Geo &, const A &a, const Lane<M, P, NP, AL> &L, double (&out)[1][M])
     {
         double f[M], w[M + 2 * HALO];
 #pragma unroll
         for (int k = 0; k < M; k++) f[k] = L.ld(0, k);
         window<M>(f, L, w);
-        op_filt<M>(w, a.C, a.tab->op[2].scale, a.tab->op[2], L, out[0]);
+        op_filt<M>(w, a.C, a.tab()->op[2].scale, a.tab()->op[2], L, out[0]);
     }
-    DEV static void store(const Geo &, const PassArgs &a, long gi, const double *v) { a.out0[gi] = v[0]; }
+    template <class A>
+    DEV static void store(const Geo &, const A &a, long gi, const double *v) { a.out0[gi] = v[0]; }
 };
 
 struct PassGauss : NoReuse {
     static constexpr int NSLOT = 1, NOUT = 1, NEARLY = 0;
-    DEV static void load(const Geo &, const PassArgs &a, long gi, double (&v)[1]) { v[0] = a.in0[gi]; }
-    template <int M, int P, bool NP, bool AL>
-    DEV static void compute(const Geo &, const PassArgs &a, const Lane<M, P, NP, AL> &L, double (&out)[1][M])
+    template <class A>
+    DEV static void load(const Geo &, const A &a, long gi, double (&v)[1]) { v[0] = a.in0[gi]; }
+    template <int M, int P, bool NP, bool AL, class A>
+    DEV static void compute(const Geo &, const A &a, const Lane<M, P, NP, AL> &L, double (&out)[1][M])
     {
         double f[M], w[M + 2 * HALO];
 #pragma unroll
@@ -78,7 +85,8 @@ struct PassGauss : NoReuse {
         window<M>(f, L, w);
         op_gauss<M>(w, a.C, out[0]);
     }
-    DEV static void store(const Geo &, const PassArgs &a, long gi, const double *v) { a.out0[gi] = v[0]; }
+    template <class A>
+    DEV static void store(const Geo &, const A &a, long gi, const double *v) { a.out0[gi] = v[0]; }
 };
 
 

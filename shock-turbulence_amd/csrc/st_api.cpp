@@ -167,6 +167,7 @@ st::PassArgs base_args(st_ctx *c)
     a.Hc = c->Hc;
     a.dQp = c->dQp;
     a.L2ep = c->L2ep;
+    a.keep_hc = 1;
     return a;
 }
 
@@ -188,14 +189,16 @@ double kind_fields(int kind, int dir, const st::PassArgs &a)
     // S, Lap e and the L2S, L4e partials in; L2S, L4e, L4S out
     case st::K_LAPSE_LAP2: return 4 + 3;
     case st::K_GAUSS_ETA: return 4;
-    // eta, C_beta, beta* mu* kappa* (written), the z-flux inputs (8 G, 4 Q), dQ 4 (read and written)
-    case st::K_GAUSS_ETA_LAST: return 2 + (a.Cb ? 1 : 0) + 3 + 8 + 4 + 8;
-    case st::K_HDIV: return 3 + 8 + 4 + 8;
+    // eta, C_beta, beta* mu* kappa* (written where kept), 12 G, 4 Q, the x and
+    // y fluxes (7 written), dQ 4 (read and written)
+    case st::K_GAUSS_ETA_LAST: return 2 + (a.Cb ? 1 : 0) + (a.keep_hc ? 3 : 0) + 12 + 4 + 7 + 8;
+    // four fluxes, dQ 4 (read and written)
+    case st::K_HDIV: return 4 + 8;
     case st::K_RKF: return 15 + 5 + 5;
     case st::K_FQ: return 10;
     case st::K_FQ_FIX: return 10;
-    // the divergence inputs (Hc, 8 G, Q), dQ, QW; QW and Q written
-    case st::K_HDIV_RKF: return 3 + 8 + 5 + 5 + 5 + 5 + 5;
+    // four fluxes, Q, dQ, QW; QW and Q written
+    case st::K_HDIV_RKF: return 4 + 5 + 5 + 5 + 5 + 5;
     // Q, G of y (written), 8 G of x and z (the four inputs of the mixed
     // terms and four more), the z and x partials, dQ (written); with the
     // artificial transport the Laplacian of e (2 partials in, the sum out),
@@ -544,6 +547,14 @@ int rk_loop(int scheme, int loop, const double **a, const double **b)
     return 0;
 }
 
+// Whether stage k of a loop is the last of the step.
+bool last_stage(int scheme, int loop, int k)
+{
+    const double *a, *b;
+    const int n = rk_loop(scheme, loop, &a, &b);
+    return k == n - 1 && (loop == 1 || !rk_loop(scheme, 1, &a, &b));
+}
+
 // Host arrays hold one instance (nfields x ni, contiguous); on the device
 // the fields of slot `slot` sit at dev + f*N + slot*ni.
 int up(st_ctx *c, double *dev, const double *host, long nfields, int slot = 0)
@@ -636,9 +647,13 @@ int seq_hyper(st_ctx *c, const st::PassArgs &base, const st::PassArgs *rk = null
     return 0;
 }
 
-// One stage body (src/lddrk4_periodic_sf.f:344-356).
-int seq_stage(st_ctx *c, const st::PassArgs &base, double ra, double rb, double dt)
+// One stage body (src/lddrk4_periodic_sf.f:344-356).  last: the coefficients
+// /HYPER/ are left in Hc (the stages before the last of a step rewrite them
+// before anything reads them).
+int seq_stage(st_ctx *c, const st::PassArgs &base0, double ra, double rb, double dt, bool last = true)
 {
+    st::PassArgs base = base0;
+    base.keep_hc = last ? 1 : 0;
     st::PassArgs a = base;
     a.rk_a = ra;
     a.rk_b = rb;
@@ -775,7 +790,7 @@ int stage_loop(st_ctx *c, double dt, double *time, int *step)
         if (!ns) break;
         // QW = 0 at the loop start (:339, :376): the first stage's alpha is 0
         // and the update then does not read QW
-        for (int k = 0; k < ns; k++) TRY(seq_stage(c, base, ra[k], rb[k], dt));
+        for (int k = 0; k < ns; k++) TRY(seq_stage(c, base, ra[k], rb[k], dt, last_stage(c->p.rk_scheme, loop, k)));
         if (time) *time = *time + dt;                        // :372, :419
     }
     if (step) *step = *step + 1;                             // :420
@@ -808,7 +823,8 @@ int batch_step(st_ctx *c)
         const double *ra, *rb;
         const int ns = rk_loop(c->p.rk_scheme, loop, &ra, &rb);
         if (!ns) break;
-        for (int k = 0; k < ns; k++) TRY(seq_stage(c, a, ra[k], rb[k], 0.0));   // (QW: as stage_loop)
+        for (int k = 0; k < ns; k++)                         // (QW: as stage_loop)
+            TRY(seq_stage(c, a, ra[k], rb[k], 0.0, last_stage(c->p.rk_scheme, loop, k)));
         const int last = loop == 1 || !rk_loop(c->p.rk_scheme, 1, &ra, &rb);
         err = st::run_clock(c->ns, c->s_run, c->s_dt, c->s_time, c->s_step, last, c->s);
         if (err != hipSuccess) return fail(c, -4, "batch clock: %s", hipGetErrorString(err));
@@ -1201,12 +1217,12 @@ namespace {
 
 // Record one stage of member m (nothing is launched); the member's passes
 // all take the M/2-point layouts of the size family.
-int group_record(st_ctx *m, const st::PassArgs &a, double ra, double rb, std::vector<Rec> &out)
+int group_record(st_ctx *m, const st::PassArgs &a, double ra, double rb, bool last, std::vector<Rec> &out)
 {
     out.clear();
     m->rec = &out;
     m->force_narrow = 1;
-    const int r = seq_stage(m, a, ra, rb, 0.0);
+    const int r = seq_stage(m, a, ra, rb, 0.0, last);
     m->rec = nullptr;
     m->force_narrow = 0;
     return r;
@@ -1252,7 +1268,7 @@ int group_step(st_group *G)
             for (int c = c0; c < 4; c++) {
                 st_ctx *m = G->m[c];
                 if (!m || !m->nact) continue;
-                if (group_record(m, a[c], ra[k], rb[k], rec[c]))
+                if (group_record(m, a[c], ra[k], rb[k], last_stage(p.rk_scheme, loop, k), rec[c]))
                     return st::set_call_error(-4, "group stage (%d points): %s", m->Mx, m->err);
                 if (rec[c].size() != rec[c0].size())
                     return st::set_call_error(-4, "group stage: members record different pass sequences");

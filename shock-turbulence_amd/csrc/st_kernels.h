@@ -20,7 +20,10 @@ struct PassArgs {
     double *L2e, *S, *Cb, *L2S, *L4e, *L4S;
     double *eta;          // 2 fields
     double *Hc;           // beta*, mu*, kappa*
-    const double *dQp;    // z and x right-hand-side partials of the first-derivative passes (2 x 5 fields)
+    // z and x right-hand-side partials of the first-derivative passes (2 x 5
+    // fields); once those are summed, the artificial fluxes of the x and y
+    // divergence (FLUX_*)
+    double *dQp;
     const double *L2ep;   // z and x partials of the Laplacian of e (2 fields)
     const double *in0;    // single-operator input
     double *out0, *out1;  // single-operator outputs
@@ -42,7 +45,7 @@ struct PassArgs {
     // and right reference states (5 each); null: no sponge in the update
     const double *spg;
     int spg_left;         // x indices below this take the left state
-    int pad3_;
+    int keep_hc;          // gauss_hdiv: write Hc (0: nothing reads it before the next stage rewrites it)
     // the tables, in the constant address space (no kernel writes them)
     __device__ __forceinline__ const __attribute__((address_space(4))) DirTab *tab() const
     {
@@ -57,6 +60,10 @@ __device__ __forceinline__ void slot_params(const PassArgs &a, int slot, PassArg
     if (a.sre) out.ph.re_inv = a.sre[slot];
     if (a.sdt) out.dt = a.sdt[slot];
 }
+
+// Fields of dQp that hold the artificial stresses and energy fluxes between
+// the z pass that forms them and the x and y passes of the divergence.
+enum FluxField { FLUX_XX, FLUX_XY, FLUX_XZ, FLUX_EX, FLUX_YY, FLUX_YZ, FLUX_EY };
 
 enum PassKind {
     K_D1, K_D2, K_FILT, K_GAUSS,

@@ -30,7 +30,7 @@ void pass_default_cfg(int kind, int dir, int *narrow, int *nt)
     case K_LAP2_LAST: c = {1, 256}; break;
     case K_LAPSE_LAP2: c = {0, 512}; break;
     case K_GAUSS_ETA: c = dir == 0 ? C{1, 1024} : C{1, 256}; break;
-    case K_GAUSS_ETA_LAST: c = {1, 1024}; break;
+    case K_GAUSS_ETA_LAST: c = {0, 512}; break;
     case K_HDIV: c = dir == 0 ? C{0, 512} : C{1, 512}; break;
     case K_HDIV_RKF: c = dir == 0 ? C{0, 512} : C{1, 256}; break;
     case K_RKF: c = {0, 256}; break;

@@ -50,7 +50,7 @@ struct Args : PassArgs {
         L4S = {b.L4S};
         eta = {b.eta};
         Hc = {b.Hc};
-        dQp = {const_cast<double *>(b.dQp)};
+        dQp = {b.dQp};
         L2ep = {const_cast<double *>(b.L2ep)};
         in0 = {const_cast<double *>(b.in0)};
         out0 = {b.out0};
@@ -119,14 +119,22 @@ struct hold_n<T, std::void_t<decltype(T::NHOLD)>> { static constexpr int value =
 
 // NLCARRY of a pass (0 when it names none): values per point that load()
 // returns after the staged and held ones and that wait in registers until
-// the memory-order phase that uses them: mid() for a pass with MID, else
-// the late store (either takes them as its last argument).  These phases
-// visit the same points per thread as the load, so a value the load phase
-// reads or derives at a point need not be read again there.
+// the late store, which takes them as its last argument.  It visits the same
+// points per thread as the load, so a value the load phase reads or derives
+// at a point need not be read again there.
 template <class T, class = void>
 struct lcarry_n { static constexpr int value = 0; };
 template <class T>
 struct lcarry_n<T, std::void_t<decltype(T::NLCARRY)>> { static constexpr int value = T::NLCARRY; };
+
+// NMF of a pass with MID (0 when it names none): global values per point
+// that mid() reads, loaded with mfetch() for MF_BATCH points before the first
+// mid() of the batch, for the same reason as NSF; mid() takes them after the
+// staged values.
+template <class T, class = void>
+struct mf_n { static constexpr int value = 0; static constexpr int batch = 1; };
+template <class T>
+struct mf_n<T, std::void_t<decltype(T::NMF)>> { static constexpr int value = T::NMF; static constexpr int batch = T::MF_BATCH; };
 
 template <class T, class = void>
 struct has_mid { static constexpr bool value = false; };
@@ -223,19 +231,33 @@ DEV void pass_body(const Geo &g, const PassArgs &a0, long tile)
     const Walk<M, P, NT> Wl(g, tile - (long)si * g.tpi, (long)slot * a.ni, tl);
     if constexpr (has_mid<PASS>::value) {
         static_assert(RE && NO == 0, "a second compute phase works on the slots");
+        constexpr int NMF = mf_n<PASS>::value, MFB = mf_n<PASS>::batch < M ? mf_n<PASS>::batch : M;
         __syncthreads();
 #pragma unroll
-        for (int r = 0; r < M; r++) {
-            int b, s;
-            const long gi = Wl.at(g, r, b, s);
-            const int li = lds_idx<M, AL>(b, s % M, s / M, P, lds_g<M>(b, NT / P));
-            double v[NS];
+        for (int r0 = 0; r0 < M; r0 += MFB) {
+            double mf[MFB][NMF > 0 ? NMF : 1];
+            if constexpr (NMF > 0) {
 #pragma unroll
-            for (int q = 0; q < NS; q++) v[q] = lds[q * ss + li];
-            if constexpr (NLC > 0) PASS::mid(g, a, gi, s, v, lc[r]);
-            else PASS::mid(g, a, gi, s, v);
+                for (int j = 0; j < MFB; j++) {
+                    if (r0 + j >= M) break;
+                    int b, s;
+                    PASS::mfetch(g, a, Wl.at(g, r0 + j, b, s), mf[j]);
+                }
+            }
 #pragma unroll
-            for (int q = 0; q < NS; q++) lds[q * ss + li] = v[q];
+            for (int j = 0; j < MFB; j++) {
+                if (r0 + j >= M) break;
+                int b, s;
+                const long gi = Wl.at(g, r0 + j, b, s);
+                const int li = lds_idx<M, AL>(b, s % M, s / M, P, lds_g<M>(b, NT / P));
+                double v[NS];
+#pragma unroll
+                for (int q = 0; q < NS; q++) v[q] = lds[q * ss + li];
+                if constexpr (NMF > 0) PASS::mid(g, a, gi, s, v, mf[j]);
+                else PASS::mid(g, a, gi, s, v);
+#pragma unroll
+                for (int q = 0; q < NS; q++) lds[q * ss + li] = v[q];
+            }
         }
         __syncthreads();
         PASS::template compute2<M, P, NP>(g, a, L);
@@ -313,9 +335,8 @@ DEV void pass_body(const Geo &g, const PassArgs &a0, long tile)
             for (int q = 0; q < NK; q++) v[NV + q] = lds[(NS - NK + q) * ss + li];
 #pragma unroll
             for (int q = 0; q < NPF; q++) v[NV + NK + q] = pf[r][q];
-            constexpr bool LCS = NLC > 0 && !has_mid<PASS>::value;
-            static_assert(!LCS || (NSF > 0 && NCR > 0), "a load carry to the store goes with store-phase fetches and a carry");
-            if constexpr (LCS) PASS::store(g, a, gi, v, cr[r], sf[j], lc[r]);
+            static_assert(NLC == 0 || (NSF > 0 && NCR > 0), "a load carry to the store goes with store-phase fetches and a carry");
+            if constexpr (NLC > 0) PASS::store(g, a, gi, v, cr[r], sf[j], lc[r]);
             else if constexpr (NSF > 0) PASS::store(g, a, gi, v, cr[r], sf[j]);
             else if constexpr (NCR > 0) PASS::store(g, a, gi, v, cr[r]);
             else PASS::store(g, a, gi, v);

@@ -27,21 +27,18 @@ struct PassHdivRkf {
     static constexpr int MIN_WAVES = 1;
     static constexpr int LOAD_UNROLL = 8;
     static constexpr int NPF = 0;
-    // the momenta and density that the fluxes read go on to the update in
-    // registers (mid reads only the energy of Q)
-    static constexpr int NLCARRY = 4;
+    // dQ, Q and QW of two points are in flight before the first is updated
+    static constexpr int NMF = 15, MF_BATCH = 2;
     template <class A>
     DEV static void prefetch(const Geo &, const A &, long, double *) {}
     template <class A>
-    DEV static void load(const Geo &g, const A &a, long gi, double (&v)[5 + NLCARRY])
+    DEV static void load(const Geo &g, const A &a, long gi, double (&v)[5])
     {
         double t[4];
         PassHyperDiv::load(g, a, gi, t);
 #pragma unroll
         for (int c = 0; c < 4; c++) v[c] = t[c];
         v[4] = 0.0;
-#pragma unroll
-        for (int c = 0; c < 4; c++) v[5 + c] = a.Q[c * a.N + gi];
     }
     template <int M, int P, bool NP, bool AL, class A>
     DEV static void compute(const Geo &g, const A &a, const Lane<M, P, NP, AL> &L, double (&o)[1][M])
@@ -49,15 +46,21 @@ struct PassHdivRkf {
         PassHyperDiv::compute<M, P, NP>(g, a, L, o);
     }
     template <class A>
-    DEV static void mid(const Geo &g, const A &a, long gi, int ix, double (&v)[5], const double *lq)
+    DEV static void mfetch(const Geo &, const A &a, long gi, double *m)
+    {
+#pragma unroll
+        for (int c = 0; c < 5; c++) {
+            const long o = c * a.N + gi;
+            m[c] = a.dQ[o];
+            m[5 + c] = a.Q[o];
+            m[10 + c] = a.rk_a == 0.0 ? 0.0 : (double)a.QW[o];
+        }
+    }
+    template <class A>
+    DEV static void mid(const Geo &g, const A &a, long gi, int ix, double (&v)[5], const double *m)
     {
         const long N = a.N;
-        double dq[5];
-        dq[0] = a.dQ[gi] + v[0];
-        dq[1] = a.dQ[N + gi] + v[1];
-        dq[2] = a.dQ[2 * N + gi] + v[2];
-        dq[3] = a.dQ[3 * N + gi];
-        dq[4] = a.dQ[4 * N + gi] + v[3];
+        const double dq[5] = {m[0] + v[0], m[1] + v[1], m[2] + v[2], m[3], m[4] + v[3]};
         // Sponge_Forcing after Hyper_RHS (src/lddrk4_nonperiodic_mf.f:462-466),
         // as k_sponge rounds it; sigma and the reference state by x index
         if (a.spg && g.dir != 0) ix = (int)((gi % a.ni) / ((long)g.My * g.Mz));
@@ -65,12 +68,11 @@ struct PassHdivRkf {
         const double *ref = a.spg ? a.spg + g.Mx + (ix < a.spg_left ? 0 : 5) : nullptr;
 #pragma unroll
         for (int c = 0; c < 5; c++) {
-            const long o = c * N + gi;
-            const double q = c < 4 ? lq[c] : (double)a.Q[o];
-            if (sg != 0.0) dq[c] = fma(-sg, q - ref[c], dq[c]);
+            const double q = m[5 + c];
+            const double d = sg != 0.0 ? fma(-sg, q - ref[c], dq[c]) : dq[c];
             // as PassFilterQ<0> (alpha = 0: QW not read)
-            const double qw = a.rk_a == 0.0 ? fma(a.dt, dq[c], 0.0) : fma(a.dt, dq[c], a.rk_a * a.QW[o]);
-            a.QW[o] = qw;
+            const double qw = a.rk_a == 0.0 ? fma(a.dt, d, 0.0) : fma(a.dt, d, a.rk_a * m[10 + c]);
+            a.QW[c * N + gi] = qw;
             v[c] = fma(a.rk_b, qw, q);
         }
     }

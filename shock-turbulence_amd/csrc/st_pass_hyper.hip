@@ -67,12 +67,20 @@ struct PassLapSELap2 {
 #pragma unroll 1
         for (int m = 0; m < 2; m++) d2_slot<M, P, NP>(a, L, m);
     }
+    // the sums so far, of all the thread's points before the first is stored
+    static constexpr int NMF = 2, MF_BATCH = 8;
     template <class A>
-    DEV static void mid(const Geo &, const A &a, long gi, int, double (&v)[2])
+    DEV static void mfetch(const Geo &, const A &a, long gi, double *m)
     {
-        const double l2s = a.L2S[gi] + v[0];       // as the accumulating D2 pass of |S| and Lap e
+        m[0] = a.L2S[gi];
+        m[1] = a.L4e[gi];
+    }
+    template <class A>
+    DEV static void mid(const Geo &, const A &a, long gi, int, double (&v)[2], const double *m)
+    {
+        const double l2s = m[0] + v[0];            // as the accumulating D2 pass of |S| and Lap e
         a.L2S[gi] = l2s;
-        a.L4e[gi] = a.L4e[gi] + v[1];
+        a.L4e[gi] = m[1] + v[1];
         v[0] = l2s;
         v[1] = 0.0;
     }
@@ -187,11 +195,18 @@ struct PassGaussEta : NoReuse {
 // ---------------------------------------------------------------------
 // The z pass of the Gaussian smoothing fused with the z pass of the
 // divergence: the smoothed eta gives the transport coefficients beta*,
-// mu*, kappa* (src/hyper_dynamic.f:303-314), which are written out for the
-// other divergence passes and, at the same point, give the z fluxes of the
-// divergence (src/hyper_rhs.f:159-491), whose D1z is added into dQ.
+// mu*, kappa* (src/hyper_dynamic.f:303-314) and, at the same point, all the
+// artificial stresses and energy fluxes (src/hyper_rhs.f:159-491).  Those of
+// the z direction are staged and their D1z added into dQ; those of x and y
+// are written for their passes, which then read four fields each instead of
+// the coefficients, eight gradients and the state.  The pass is bound by
+// memory: 34 fields a point (37 with the coefficients written, which only
+// the last stage of a step needs).  256^3: this pass 0.74 -> 0.86 ms at 26 ->
+// 34 fields, the x pass 0.69 -> 0.34 ms (23 -> 12), the y pass 0.96 -> 0.80
+// ms (36 -> 29).
 //   compute   Gaussian along z of the two eta fields
-//   mid       per point: beta*, mu*, kappa* (written), the staged z fluxes
+//   mid       per point: beta*, mu*, kappa*, the x and y fluxes (written),
+//             the staged z fluxes
 //   compute2  D1z of the fluxes
 // ---------------------------------------------------------------------
 struct PassGaussHdiv {
@@ -225,19 +240,49 @@ struct PassGaussHdiv {
             for (int k = 0; k < M; k++) L.st(m, k, r[k]);
         }
     }
+    // the 12 gradients, the momenta and density, C_beta
+    static constexpr int NMF = 17, MF_BATCH = 2;
     template <class A>
-    DEV static void mid(const Geo &g, const A &a, long gi, int, double (&v)[4])
+    DEV static void mfetch(const Geo &, const A &a, long gi, double *m)
+    {
+#pragma unroll
+        for (int c = 0; c < 12; c++) m[c] = a.G[c * a.N + gi];
+#pragma unroll
+        for (int c = 0; c < 4; c++) m[12 + c] = a.Q[c * a.N + gi];
+        // constant C_beta = 1 without the sensor (src/hyper_routines.f:99-101,204)
+        m[16] = a.Cb ? (double)a.Cb[gi] : 1.0;
+    }
+    template <class A>
+    DEV static void mid(const Geo &, const A &a, long gi, int, double (&v)[4], const double *m)
     {
         const Phys &ph = a.ph;
         const long N = a.N;
-        // beta*; constant C_beta = 1 without the sensor (src/hyper_routines.f:99-101,204)
-        const double beta = (a.Cb ? a.Cb[gi] : 1.0) * v[0] * ph.dx6;
+        const double beta = m[16] * v[0] * ph.dx6;
         const double mu = ph.cmu * v[0] * ph.dx6;
         const double kap = ph.ck * v[1] * ph.dx5;
-        a.Hc[gi] = beta;
-        a.Hc[N + gi] = mu;
-        a.Hc[2 * N + gi] = kap;
-        PassHyperDiv::fluxes<false>(g, a, gi, beta, mu, kap, v);
+        if (a.keep_hc) {
+            a.Hc[gi] = beta;
+            a.Hc[N + gi] = mu;
+            a.Hc[2 * N + gi] = kap;
+        }
+        const double gxx = m[0], gyy = m[4], gzz = m[8];
+        const double dil = gxx + gyy + gzz;
+        const double uh = m[12] / m[15], vh = m[13] / m[15], wh = m[14] / m[15];
+        const double tt = 2.0 / 3.0;
+        const double bulkterm = (beta - tt * mu) * dil;
+        const double xx = 2.0 * mu * gxx + bulkterm, yy = 2.0 * mu * gyy + bulkterm, zz = 2.0 * mu * gzz + bulkterm;
+        const double xy = mu * (m[3] + m[1]), xz = mu * (m[6] + m[2]), yz = mu * (m[7] + m[5]);
+        a.dQp[FLUX_XX * N + gi] = xx;
+        a.dQp[FLUX_XY * N + gi] = xy;
+        a.dQp[FLUX_XZ * N + gi] = xz;
+        a.dQp[FLUX_EX * N + gi] = uh * xx + vh * xy + wh * xz + kap * m[9];
+        a.dQp[FLUX_YY * N + gi] = yy;
+        a.dQp[FLUX_YZ * N + gi] = yz;
+        a.dQp[FLUX_EY * N + gi] = uh * xy + vh * yy + wh * yz + kap * m[10];
+        v[0] = xz;
+        v[1] = yz;
+        v[2] = zz;
+        v[3] = uh * xz + vh * yz + wh * zz + kap * m[11];
     }
     template <int M, int P, bool NP, bool AL, class A>
     DEV static void compute2(const Geo &g, const A &a, const Lane<M, P, NP, AL> &L)

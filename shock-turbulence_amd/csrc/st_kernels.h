@@ -108,6 +108,15 @@ hipError_t launch_hyper_ragged(int kind, const RaggedSpec &sp, hipStream_t s);
 hipError_t launch_hdivrk_ragged(int kind, const RaggedSpec &sp, hipStream_t s);
 hipError_t launch_filter_ragged(int kind, const RaggedSpec &sp, hipStream_t s);
 
+// Points of a launch from which its passes stream past the caches: the 57
+// fields of a stage are then 0.7 GB, well over the 256 MB of the last-level
+// cache, so nothing that one pass leaves there is found by the next.  Stage
+// times without and with streaming loads and stores, us: 64^3 x 4 (1.05 M
+// points) 418 / 421, 256 x 64 x 64 402 / 408, 112^3 (1.4 M) 618 / 615, 48^3 x
+// 16 (1.8 M) 696 / 677, 128^3 800 / 780, 64^3 x 12 1105 / 1041, 256^3 6072 /
+// 5634.
+constexpr long STREAM_POINTS = 3L << 19;
+
 // Default launch layout of a pass kind: narrow = 1 uses the tables with half
 // the points per lane (twice the lanes per line); nt = threads per workgroup.
 void pass_default_cfg(int kind, int dir, int *narrow, int *nt);

@@ -14,28 +14,33 @@ namespace st {
 // ---------------------------------------------------------------------
 // field access of a pass
 // ---------------------------------------------------------------------
-// NT: streaming (non-temporal) loads and stores.
-template <bool NT>
+// ST: streaming (non-temporal) loads (STREAM_LOADS) and stores (STREAM_STORES).
+enum : int { STREAM_LOADS = 1, STREAM_STORES = 2, STREAM_Y = 4 };
+template <int ST>
 struct GRef {
     double *p;
-    DEV operator double() const { return NT ? __builtin_nontemporal_load(p) : *p; }
+    DEV operator double() const
+    {
+        if constexpr (ST & STREAM_LOADS) return __builtin_nontemporal_load(p);
+        else return *p;
+    }
     DEV void operator=(double v) const
     {
-        if constexpr (NT) __builtin_nontemporal_store(v, p);
+        if constexpr (ST & STREAM_STORES) __builtin_nontemporal_store(v, p);
         else *p = v;
     }
 };
-template <bool NT>
+template <int ST>
 struct GPtr {
     double *p;
-    DEV GRef<NT> operator[](long i) const { return {p + i}; }
+    DEV GRef<ST> operator[](long i) const { return {p + i}; }
     DEV explicit operator bool() const { return p != nullptr; }
 };
 
 // The arguments as a pass sees them: every field through GPtr.
-template <bool NT>
+template <int ST>
 struct Args : PassArgs {
-    GPtr<NT> Q, QW, dQ, G, L2e, S, Cb, L2S, L4e, L4S, eta, Hc, dQp, L2ep, in0, out0, out1;
+    GPtr<ST> Q, QW, dQ, G, L2e, S, Cb, L2S, L4e, L4S, eta, Hc, dQp, L2ep, in0, out0, out1;
     DEV Args(const PassArgs &b) : PassArgs(b)
     {
         Q = {b.Q};
@@ -136,6 +141,19 @@ struct mf_n { static constexpr int value = 0; static constexpr int batch = 1; };
 template <class T>
 struct mf_n<T, std::void_t<decltype(T::NMF)>> { static constexpr int value = T::NMF; static constexpr int batch = T::MF_BATCH; };
 
+// STREAM of a pass (0 when it names none): whether its loads and stores go
+// past the caches (non-temporal) on a large grid, and whether it sweeps y.
+// The y passes read and write whole lines once (256^3: the gradient pass 1.00
+// -> 0.93 ms, the divergence and update 0.80 -> 0.70, the Laplacian and
+// Gaussian 0.27 -> 0.19); a strided pass gains only with tiles of 16 lines or
+// more, whose rows are whole 128-byte lines (narrower rows share a line
+// between tiles: the x gradient pass on 8-line tiles 0.58 -> 0.69 ms).  The
+// filters and the z gradient pass, on narrow tiles, name none.
+template <class T, class = void>
+struct stream_n { static constexpr int value = 0; };
+template <class T>
+struct stream_n<T, std::void_t<decltype(T::STREAM)>> { static constexpr int value = T::STREAM; };
+
 template <class T, class = void>
 struct has_mid { static constexpr bool value = false; };
 template <class T>
@@ -156,7 +174,7 @@ struct has_mid<T, std::void_t<decltype(T::MID)>> { static constexpr bool value =
 // A REUSE pass with NCARRY > 0 gets a per-point register array in both
 // store phases (same points per thread): store_early() fills it, store()
 // reads it, so early results can feed the late store without a slot.
-template <int M, int P, int NT, bool NP, class PASS>
+template <int M, int P, int NT, bool NP, class PASS, int ST = 0>
 DEV void pass_body(const Geo &g, const PassArgs &a0, long tile)
 {
     extern __shared__ double lds[];
@@ -181,7 +199,7 @@ DEV void pass_body(const Geo &g, const PassArgs &a0, long tile)
     if (a0.act && !a0.act[slot]) return;          // uniform per workgroup, before any barrier
     PassArgs ap;
     slot_params(a0, slot, ap);
-    const Args<false> a(ap);
+    const Args<ST> a(ap);
     const Walk<M, P, NT> W(g, tile - (long)si * g.tpi, (long)slot * a.ni, threadIdx.x);
     constexpr int ss = NT * M;           // slot size: B*M*P with B*P = NT
 
@@ -344,11 +362,13 @@ DEV void pass_body(const Geo &g, const PassArgs &a0, long tile)
     }
 }
 
-template <int M, int P, int NT, bool NP, class PASS>
+template <int M, int P, int NT, bool NP, class PASS, int ST>
 __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(PASS::MIN_WAVES)))
 k_pass(Geo g, PassArgs a0)
 {
-    pass_body<M, P, NT, NP, PASS>(g, a0, tile_of(g, blockIdx.x));
+    // a streaming y pass reads no line twice and takes the tiles as they come
+    const long tile = (ST & STREAM_Y) ? (long)blockIdx.x : tile_of(g, blockIdx.x);
+    pass_body<M, P, NT, NP, PASS, ST>(g, a0, tile);
 }
 
 // Passes whose early outputs have their own slots.
@@ -379,8 +399,8 @@ DEV void qown(const Lane<M, P, NP, AL> &L, int k, double &q1, double &q2, double
     q5 = L.ld(4, k);
 }
 
-template <bool NT>
-DEV void upd(GRef<NT> p, double v, bool first)
+template <int ST>
+DEV void upd(GRef<ST> p, double v, bool first)
 {
     p = first ? v : p + v;
 }
@@ -389,21 +409,34 @@ DEV void upd(GRef<NT> p, double v, bool first)
 // ---------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------
-template <int M, int P, int NT, bool NP, class PASS>
-static hipError_t launch_t(const Geo &g, const PassArgs &a, hipStream_t s)
+template <int M, int P, int NT, bool NP, class PASS, int ST>
+static hipError_t launch_s(const Geo &g, const PassArgs &a, size_t lds, hipStream_t s)
 {
-    const size_t lds = (size_t)pass_slots<PASS>() * NT * M * sizeof(double);
-    if (lds > 160 * 1024) return hipErrorInvalidValue;
-    if (a.dry) return hipSuccess;
     static size_t lds_set = 0;
     if (lds > 64 * 1024 && lds > lds_set) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_pass<M, P, NT, NP, PASS>),
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_pass<M, P, NT, NP, PASS, ST>),
                                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
         lds_set = lds;
     }
-    hipLaunchKernelGGL((k_pass<M, P, NT, NP, PASS>), dim3((unsigned)g.ntiles), dim3(NT), lds, s, g, a);
+    hipLaunchKernelGGL((k_pass<M, P, NT, NP, PASS, ST>), dim3((unsigned)g.ntiles), dim3(NT), lds, s, g, a);
     return hipGetLastError();
+}
+
+template <int M, int P, int NT, bool NP, class PASS>
+static hipError_t launch_t(const Geo &g, const PassArgs &a, hipStream_t s)
+{
+    constexpr size_t lds = (size_t)pass_slots<PASS>() * NT * M * sizeof(double);
+    if constexpr (lds > 160 * 1024) {
+        return hipErrorInvalidValue;
+    } else {
+        if (a.dry) return hipSuccess;
+        constexpr int ST = stream_n<PASS>::value;
+        if constexpr (ST != 0 && ((ST & STREAM_Y) || NT / P >= 16)) {
+            if (a.ni * a.nslot >= STREAM_POINTS) return launch_s<M, P, NT, NP, PASS, ST>(g, a, lds, s);
+        }
+        return launch_s<M, P, NT, NP, PASS, 0>(g, a, lds, s);
+    }
 }
 
 // The lane layouts (M points per lane, P lanes per line) that

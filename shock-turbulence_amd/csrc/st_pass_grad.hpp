@@ -67,6 +67,7 @@ struct PassGrad {
     // dw/dz) and the viscosity reach the store after the late results
     static constexpr int NKEEP = CROSS ? NMX + 1 : 0;
     static constexpr int MIN_WAVES = MW;
+    static constexpr int STREAM = DIR == 2 ? 0 : STREAM_LOADS | STREAM_STORES | (DIR == 1 ? STREAM_Y : 0);
     static constexpr int LOAD_UNROLL = 8;
     static constexpr int NPF = 0;
     // the additive LDS layout for the x and y sweeps (fewer address

@@ -17,6 +17,7 @@ namespace st {
 // them again from Hc, eight gradients and the state, and divides nowhere.
 // ---------------------------------------------------------------------
 struct PassHyperDiv {
+    static constexpr int STREAM = STREAM_LOADS;
     static constexpr int NSLOT = 4, NOUT = 0, NEARLY = 4;
     static constexpr bool REUSE = true;
     static constexpr int MIN_WAVES = 1;

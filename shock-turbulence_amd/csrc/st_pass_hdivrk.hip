@@ -24,6 +24,7 @@ struct PassHdivRkf {
     static constexpr int NSLOT = 5, NOUT = 0, NEARLY = 5;
     static constexpr bool REUSE = true;
     static constexpr bool MID = true;
+    static constexpr int STREAM = STREAM_LOADS | STREAM_STORES | STREAM_Y;
     static constexpr int MIN_WAVES = 1;
     static constexpr int LOAD_UNROLL = 8;
     static constexpr int NPF = 0;

@@ -8,6 +8,7 @@ namespace st {
 // to the z pass's partial in L4S.
 // ---------------------------------------------------------------------
 struct PassLap2 : NoReuse {
+    static constexpr int STREAM = STREAM_LOADS;
     static constexpr int NSLOT = 1, NOUT = 1, NEARLY = 0;
     template <class A>
     DEV static void load(const Geo &, const A &a, long gi, double (&v)[1]) { v[0] = a.L2S[gi]; }
@@ -47,6 +48,7 @@ DEV void d2_slot(const A &a, const Lane<M, P, NP, AL> &L, int m)
 //   store     L4S = D2z L2S (the first direction of the second Laplacian)
 // ---------------------------------------------------------------------
 struct PassLapSELap2 {
+    static constexpr int STREAM = STREAM_LOADS;
     static constexpr int NSLOT = 2, NOUT = 0, NEARLY = 1;
     static constexpr bool REUSE = true;
     static constexpr bool MID = true;
@@ -105,6 +107,7 @@ struct PassLapSELap2 {
 //   store     eta
 // ---------------------------------------------------------------------
 struct PassLap2Gauss {
+    static constexpr int STREAM = STREAM_LOADS | STREAM_STORES | STREAM_Y;
     static constexpr int NSLOT = 2, NOUT = 0, NEARLY = 2;
     static constexpr bool REUSE = true;
     static constexpr bool MID = true;
@@ -165,6 +168,7 @@ struct PassLap2Gauss {
 // PassLap2Gauss, z in PassGaussHdiv).
 // ---------------------------------------------------------------------
 struct PassGaussEta : NoReuse {
+    static constexpr int STREAM = STREAM_LOADS;
     static constexpr int NSLOT = 2, NOUT = 2, NEARLY = 0;
     template <class A>
     DEV static void load(const Geo &, const A &a, long gi, double (&v)[2])
@@ -210,6 +214,7 @@ struct PassGaussEta : NoReuse {
 //   compute2  D1z of the fluxes
 // ---------------------------------------------------------------------
 struct PassGaussHdiv {
+    static constexpr int STREAM = STREAM_LOADS | STREAM_STORES;
     static constexpr int NSLOT = 4, NOUT = 0, NEARLY = 4;
     static constexpr bool REUSE = true;
     static constexpr bool MID = true;

@@ -13,6 +13,7 @@ namespace st {
 // ---------------------------------------------------------------------
 template <bool ACC>
 struct PassLapSE {
+    static constexpr int STREAM = ACC ? STREAM_LOADS | STREAM_Y : STREAM_LOADS;
     static constexpr int NSLOT = 2, NOUT = 0, NEARLY = 2;
     static constexpr bool REUSE = true;
     static constexpr int MIN_WAVES = 1;

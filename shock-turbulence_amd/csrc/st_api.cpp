@@ -288,31 +288,6 @@ extern "C" int st_batch_create(const st_grid *grid, const st_params *params, int
     std::memset(c->prof_ms, 0, sizeof(c->prof_ms));
     std::memset(c->prof_cnt, 0, sizeof(c->prof_cnt));
     std::memset(c->prof_fields, 0, sizeof(c->prof_fields));
-    // launch layouts; ST_NARROW / ST_NT512 / ST_NT1024 (bit masks over pass
-    // kinds) and ST_NT_<kind> (per direction) override the defaults
-    {
-        const char *en = getenv("ST_NARROW"), *et = getenv("ST_NT512"), *eu = getenv("ST_NT1024");
-        for (int k = 0; k < NKIND; k++) {
-            for (int d = 0; d < 3; d++) {
-                st::pass_default_cfg(k, d, &c->cfg_narrow[k][d], &c->cfg_nt[k][d]);
-                if (et) c->cfg_nt[k][d] = ((strtoul(et, nullptr, 0) >> k) & 1) ? 512 : 256;
-                if (eu && ((strtoul(eu, nullptr, 0) >> k) & 1)) c->cfg_nt[k][d] = 1024;
-            }
-            if (en)
-                for (int d = 0; d < 3; d++) c->cfg_narrow[k][d] = (int)((strtoul(en, nullptr, 0) >> k) & 1);
-            // ST_NT_<k> = "nx,ny,nz": tile threads of pass kind k per direction
-            char var[32];
-            snprintf(var, sizeof(var), "ST_NT_%d", k);
-            if (const char *ev = getenv(var)) {
-                int v[3];
-                if (sscanf(ev, "%d,%d,%d", &v[0], &v[1], &v[2]) == 3)
-                    for (int d = 0; d < 3; d++)
-                        if (v[d] == 256 || v[d] == 512 || v[d] == 1024) c->cfg_nt[k][d] = v[d];
-            }
-        }
-    }
-    if (grid->nonperiodic_x && !getenv("ST_NT1024"))
-        for (int k = 0; k < NKIND; k++) c->cfg_nt[k][0] = 256;   // boundary tables cost registers
     const int n[3] = {c->Mx, c->My, c->Mz};
     const double period[3] = {grid->period_x, grid->period_y, grid->period_z};
     const double start[3] = {grid->x_start, grid->y_start, grid->z_start};
@@ -399,6 +374,31 @@ extern "C" int st_batch_create(const st_grid *grid, const st_params *params, int
                 return -2;
             }
     }
+    // launch layouts; ST_NARROW / ST_NT512 / ST_NT1024 (bit masks over pass
+    // kinds) and ST_NT_<kind> (per direction) override the defaults
+    {
+        const char *en = getenv("ST_NARROW"), *et = getenv("ST_NT512"), *eu = getenv("ST_NT1024");
+        for (int k = 0; k < NKIND; k++) {
+            for (int d = 0; d < 3; d++) {
+                st::pass_default_cfg(k, d, c->th[d], c->ni, c->N, &c->cfg_narrow[k][d], &c->cfg_nt[k][d]);
+                if (et) c->cfg_nt[k][d] = ((strtoul(et, nullptr, 0) >> k) & 1) ? 512 : 256;
+                if (eu && ((strtoul(eu, nullptr, 0) >> k) & 1)) c->cfg_nt[k][d] = 1024;
+            }
+            if (en)
+                for (int d = 0; d < 3; d++) c->cfg_narrow[k][d] = (int)((strtoul(en, nullptr, 0) >> k) & 1);
+            // ST_NT_<k> = "nx,ny,nz": tile threads of pass kind k per direction
+            char var[32];
+            snprintf(var, sizeof(var), "ST_NT_%d", k);
+            if (const char *ev = getenv(var)) {
+                int v[3];
+                if (sscanf(ev, "%d,%d,%d", &v[0], &v[1], &v[2]) == 3)
+                    for (int d = 0; d < 3; d++)
+                        if (v[d] == 256 || v[d] == 512 || v[d] == 1024) c->cfg_nt[k][d] = v[d];
+            }
+        }
+    }
+    if (grid->nonperiodic_x && !getenv("ST_NT1024"))
+        for (int k = 0; k < NKIND; k++) c->cfg_nt[k][0] = 256;   // boundary tables cost registers
     hipError_t e;
     if ((e = hipStreamCreateWithFlags(&c->s, hipStreamNonBlocking)) != hipSuccess) {
         fail(c, -3, "hipStreamCreate: %s", hipGetErrorString(e));

@@ -117,9 +117,11 @@ hipError_t launch_filter_ragged(int kind, const RaggedSpec &sp, hipStream_t s);
 // 5634.
 constexpr long STREAM_POINTS = 3L << 19;
 
-// Default launch layout of a pass kind: narrow = 1 uses the tables with half
-// the points per lane (twice the lanes per line); nt = threads per workgroup.
-void pass_default_cfg(int kind, int dir, int *narrow, int *nt);
+// Default launch shape of a pass: narrow = 1 uses the tables with half the
+// points per lane (twice the lanes per line); nt = threads per workgroup.
+// wide: the tables with all points per lane; ni and N: points per instance
+// and of all the context's instances.
+void pass_default_cfg(int kind, int dir, const DirTab &wide, long ni, long N, int *narrow, int *nt);
 hipError_t run_pass(int kind, const DirTab &t, int nt, int dir, int My, int Mz, int Mx, const PassArgs &a, hipStream_t s);
 // per translation unit (st_pass_*.hip)
 hipError_t launch_ops(int kind, const DirTab &t, int nt, int dir, int My, int Mz, int Mx, const PassArgs &a, hipStream_t s);

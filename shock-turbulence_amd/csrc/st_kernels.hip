@@ -14,32 +14,33 @@
 
 namespace st {
 
-void pass_default_cfg(int kind, int dir, int *narrow, int *nt)
+// Launch shape of a pass: the lane layout (wide: M points per lane on P lanes;
+// narrow: M/2 on 2P) and the threads per workgroup.  Measured with each pass
+// varied in turn and the whole stage timed (us per stage, old -> new shapes).
+// Grids below STREAM_POINTS live in the caches and launch few workgroups: the
+// narrow layout halves each lane's serial work and 256-thread tiles give the
+// most workgroups (64^3 190 -> 153, 48^3 149 -> 117, 32^3 113 -> 88, 96^3 410
+// -> 353).  Larger grids are bound by memory: unit-stride (y) passes keep the
+// narrow layout and 256 threads; strided passes take the layout of 32 lanes
+// per line and tiles of 16 lines, whose rows are whole 128-byte lines that can
+// stream (256^3: x gradient 5579 -> 5465, z Gaussian and divergence 5476 ->
+// 5405); but for the passes with much arithmetic per point, the z gradient
+// (its two-round form where it exists, else narrow) and the filters, 256
+// threads, more than one workgroup per CU, do better (256^3 filter z 5382
+// against 5447).  The layout decides the rounding, so it depends on the
+// instance alone and not on how many share the launch.
+void pass_default_cfg(int kind, int dir, const DirTab &wide, long ni, long N, int *narrow, int *nt)
 {
-    // Chosen by st_autotune at 256^3 (per pass and direction): wider tiles
-    // (more lines, so longer unit-stride rows in the strided x and z sweeps)
-    // where the pass's registers allow the waves; M/2 points per lane
-    // ("narrow") where the pass holds many fields in registers.
-    struct C { int n, t; };
-    C c = {0, 256};
-    switch (kind) {
-    case K_GRAD: c = {0, 256}; break;
-    case K_GRAD_CROSS: c = {1, 256}; break;
-    case K_LAPSE: c = dir == 1 ? C{1, 512} : C{0, 512}; break;
-    case K_LAP2: c = {0, 512}; break;
-    case K_LAP2_LAST: c = {1, 256}; break;
-    case K_LAPSE_LAP2: c = {0, 512}; break;
-    case K_GAUSS_ETA: c = dir == 0 ? C{1, 1024} : C{1, 256}; break;
-    case K_GAUSS_ETA_LAST: c = {0, 512}; break;
-    case K_HDIV: c = dir == 0 ? C{0, 512} : C{1, 512}; break;
-    case K_HDIV_RKF: c = dir == 0 ? C{0, 512} : C{1, 256}; break;
-    case K_RKF: c = {0, 256}; break;
-    case K_FQ: c = {0, 256}; break;
-    case K_FQ_FIX: c = {0, 256}; break;
-    default: break;
+    *narrow = 1;
+    *nt = 256;
+    const bool split = wide.M % 2 == 0 && 2 * wide.P <= 64;       // a narrow layout exists
+    const bool compute = kind == K_FQ || kind == K_FQ_FIX || kind == K_GRAD;
+    if (dir != 1 && ni >= STREAM_POINTS) {
+        *narrow = kind == K_GRAD && dir == 2 ? !(wide.M == 8 && wide.P == 32) : wide.P < 32;
+        if (kind == K_D1 || kind == K_D2 || kind == K_FILT || kind == K_GAUSS) *narrow = 0;
     }
-    *narrow = c.n;
-    *nt = c.t;
+    const int P = *narrow && split ? 2 * wide.P : wide.P;
+    if (dir != 1 && N >= STREAM_POINTS && !(compute && !(kind == K_GRAD && dir == 0))) *nt = P <= 16 ? 256 : P == 32 ? 512 : 1024;
 }
 
 hipError_t run_pass(int kind, const DirTab &t, int nt, int dir, int My, int Mz, int Mx, const PassArgs &a, hipStream_t s)

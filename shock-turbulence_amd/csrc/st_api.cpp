@@ -19,6 +19,7 @@ namespace {
 
 constexpr int NKIND = 24;          // pass kinds + reductions + fills
 constexpr int KIND_RED = 21, KIND_FILL = 22;
+constexpr int MARCH_CHUNK = 256;   // steps of st_march between host synchronisations
 static_assert(st::K_NPASS <= KIND_RED, "pass kinds overlap the other timed kinds");
 
 // Fields read + written per point by one launch of each kind (RMW counts
@@ -69,6 +70,8 @@ struct st_ctx {
     std::vector<int> act_h;
     int nact = 0;                   // active slots, listed in s_list (launch grids cover these only)
     std::vector<hipGraphExec_t> graphs;   // one batch step, captured per active-slot count
+    double *m_clk = nullptr;        // clock and dts of st_march (device), and its pinned host copy
+    double *m_clk_h = nullptr;
     double *spg = nullptr;          // sponge: sigma per x index, then the left and right reference states
     int spg_left = 0;               // x indices [0, spg_left) take the left reference state
     int use_graph = 1;
@@ -415,6 +418,8 @@ extern "C" int st_batch_create(const st_grid *grid, const st_params *params, int
         (e = hipMalloc(&c->td, sizeof(st::DirTab) * 6)) != hipSuccess ||
         (e = hipMalloc(&c->red, sizeof(double) * c->red_n)) != hipSuccess ||
         (e = hipHostMalloc(&c->red_h, sizeof(double) * c->red_n)) != hipSuccess ||
+        (e = hipMalloc(&c->m_clk, sizeof(double) * (5 + MARCH_CHUNK))) != hipSuccess ||
+        (e = hipHostMalloc(&c->m_clk_h, sizeof(double) * (5 + MARCH_CHUNK))) != hipSuccess ||
         (e = hipMalloc(&sp, ns * (6 * sizeof(int) + 4 * sizeof(double)))) != hipSuccess) {
         fail(c, -3, "device allocation: %s", hipGetErrorString(e));
         *out = c;
@@ -482,6 +487,8 @@ extern "C" void st_ctx_destroy(st_ctx *c)
     if (c->td) (void)hipFree(c->td);
     if (c->red) (void)hipFree(c->red);
     if (c->red_h) (void)hipHostFree(c->red_h);
+    if (c->m_clk) (void)hipFree(c->m_clk);
+    if (c->m_clk_h) (void)hipHostFree(c->m_clk_h);
     if (c->s) (void)hipStreamDestroy(c->s);
     delete c;
 }
@@ -649,12 +656,15 @@ int seq_hyper(st_ctx *c, const st::PassArgs &base, const st::PassArgs *rk = null
 
 // One stage body (src/lddrk4_periodic_sf.f:344-356).  last: the coefficients
 // /HYPER/ are left in Hc (the stages before the last of a step rewrite them
-// before anything reads them).
-int seq_stage(st_ctx *c, const st::PassArgs &base0, double ra, double rb, double dt, bool last = true)
+// before anything reads them).  guard: a run flag for the passes that write
+// the state alone (the others then start without waiting for a flag).
+int seq_stage(st_ctx *c, const st::PassArgs &base0, double ra, double rb, double dt, bool last = true,
+              const int *guard = nullptr)
 {
     st::PassArgs base = base0;
     base.keep_hc = last ? 1 : 0;
     st::PassArgs a = base;
+    if (guard) a.act = guard;
     a.rk_a = ra;
     a.rk_b = rb;
     a.dt = dt;
@@ -810,11 +820,10 @@ int batch_step(st_ctx *c)
     a.act = c->s_act;
     int nb = 0;
     double *pc = c->red, *pt = c->red + (long)st::reduce_blocks(c->ni) * c->ns * 2;
-    hipError_t err = st::run_reduce(0, a, pc, &nb, c->s);
-    if (err == hipSuccess && c->p.hyper_param == 1) err = st::run_reduce(1, a, pt, &nb, c->s);
+    hipError_t err = st::run_cfl_tstep(a, pc, c->p.hyper_param == 1 ? pt : nullptr, &nb, c->s);
     if (err == hipSuccess)
         err = st::run_dt(pc, pt, nb, c->ns, c->s_act, c->s_target, c->s_step, c->p.cfl_cal, c->p.hyper_param,
-                         c->g.nonperiodic_x ? 1 : 0, c->s_run, c->s_dt, c->s_dtlast, c->s);
+                         c->g.nonperiodic_x ? 1 : 0, c->s_run, c->s_dt, c->s_dtlast, nullptr, 0, c->s);
     if (err != hipSuccess) return fail(c, -4, "batch dt: %s", hipGetErrorString(err));
     a.act = c->s_run;
     a.sre = c->s_re;
@@ -1068,19 +1077,57 @@ extern "C" int st_step(st_ctx *c, double dt, double *time, int *step)
     return 0;
 }
 
+// March of one run with its dt formed on the device, as a batch's: no host
+// round trip between the steps (each cost two synchronising copies).  The
+// run's clock lives in its own device block (a batch's slot 0 keeps its own);
+// the dts come back once per MARCH_CHUNK steps.
 extern "C" int st_march(st_ctx *c, int nsteps, double *time, int *step, double *dt_out)
 {
     if (!c || !time || !step) return -1;
-    for (int it = 0; it < nsteps; it++) {
-        double stab, resv, dt;
-        TRY(st_cfl(c, &stab, &resv));
-        TRY(st_tstep(c, resv, *step, &dt));
-        if (!(dt > 0.0) || !std::isfinite(dt)) return fail(c, -5, "non-finite or non-positive dt %g at step %d", dt, *step);
-        TRY(stage_loop(c, dt, time, step));
-        if (dt_out) dt_out[it] = dt;
+    st::PassArgs a = base_args(c);
+    double *tm = c->m_clk, *dt = c->m_clk + 1, *dt_last = c->m_clk + 2;
+    int *ints = (int *)(c->m_clk + 3);
+    int *act = ints, *run = ints + 1, *target = ints + 2, *stepc = ints + 3;
+    double *hist = c->m_clk + 5;
+    a.sdt = dt;
+    const int hyper = c->p.hyper_param, first = c->g.nonperiodic_x ? 1 : 0;
+    double *pc = c->red, *pt = c->red + (long)st::reduce_blocks(c->ni) * c->ns * 2;
+    for (int done = 0; done < nsteps;) {
+        const int n = nsteps - done < MARCH_CHUNK ? nsteps - done : MARCH_CHUNK;
+        const int step0 = *step;
+        hipError_t err = st::run_clock_set(act, target, stepc, tm, n, step0, *time, c->s);
+        if (err != hipSuccess) return fail(c, -4, "march clock: %s", hipGetErrorString(err));
+        for (int it = 0; it < n; it++) {
+            int nb = 0;
+            Event e;
+            if (c->prof) prof_begin(c, KIND_RED * 3, e);
+            err = st::run_cfl_tstep(base_args(c), pc, hyper == 1 ? pt : nullptr, &nb, c->s);
+            if (err == hipSuccess)
+                err = st::run_dt(pc, pt, nb, 1, act, target, stepc, c->p.cfl_cal, hyper, first, run, dt, dt_last, hist,
+                                 step0, c->s);
+            if (c->prof) prof_end(c, e);
+            if (err != hipSuccess) return fail(c, -4, "march dt: %s", hipGetErrorString(err));
+            for (int loop = 0; loop < 2; loop++) {
+                const double *ra, *rb;
+                const int ns = rk_loop(c->p.rk_scheme, loop, &ra, &rb);
+                if (!ns) break;
+                for (int k = 0; k < ns; k++)                 // (QW: as stage_loop)
+                    TRY(seq_stage(c, a, ra[k], rb[k], 0.0, last_stage(c->p.rk_scheme, loop, k), run));
+                err = st::run_clock(1, run, dt, tm, stepc, last_stage(c->p.rk_scheme, loop, ns - 1), c->s);
+                if (err != hipSuccess) return fail(c, -4, "march clock: %s", hipGetErrorString(err));
+            }
+        }
+        HIPCHK(c, hipMemcpyAsync(c->m_clk_h, c->m_clk, sizeof(double) * (5 + n), hipMemcpyDeviceToHost, c->s));
+        HIPCHK(c, hipStreamSynchronize(c->s));
+        if (c->prof) prof_collect(c);
+        *time = c->m_clk_h[0];
+        *step = ((const int *)(c->m_clk_h + 3))[3];
+        const double *d = c->m_clk_h + 5;
+        for (int it = 0; it < *step - step0 && dt_out; it++) dt_out[done + it] = d[it];
+        if (*step - step0 < n)
+            return fail(c, -5, "non-finite or non-positive dt %g at step %d", d[*step - step0], *step);
+        done += n;
     }
-    HIPCHK(c, hipStreamSynchronize(c->s));
-    if (c->prof) prof_collect(c);
     return 0;
 }
 
@@ -1247,11 +1294,10 @@ int group_step(st_group *G)
         b.act = m->s_act;
         int nb = 0;
         double *pc = m->red, *pt = m->red + (long)st::reduce_blocks(m->ni) * m->ns * 2;
-        err = st::run_reduce(0, b, pc, &nb, G->s);
-        if (err == hipSuccess && m->p.hyper_param == 1) err = st::run_reduce(1, b, pt, &nb, G->s);
+        err = st::run_cfl_tstep(b, pc, m->p.hyper_param == 1 ? pt : nullptr, &nb, G->s);
         if (err == hipSuccess)
             err = st::run_dt(pc, pt, nb, m->ns, m->s_act, m->s_target, m->s_step, m->p.cfl_cal, m->p.hyper_param, 0,
-                             m->s_run, m->s_dt, m->s_dtlast, G->s);
+                             m->s_run, m->s_dt, m->s_dtlast, nullptr, 0, G->s);
         if (err != hipSuccess) return st::set_call_error(-4, "group dt (%d points): %s", m->Mx, hipGetErrorString(err));
         b.act = m->s_run;
         b.sre = m->s_re;

@@ -146,7 +146,11 @@ hipError_t run_fill_slots(double *p, int nfields, long N, long ni, int nslot, co
 hipError_t run_fixp(const PassArgs &a, double *Qx, hipStream_t s);
 hipError_t run_dt(const double *pc, const double *pt, int nb, int nslot, const int *active, const int *target,
                   const int *stepc, double cfl_cal, int hyper, int first_step, int *run, double *dt, double *dt_last,
-                  hipStream_t s);
+                  double *hist, int hist0, hipStream_t s);
+// the partials of both (pt null: of the CFL numbers alone)
+hipError_t run_cfl_tstep(const PassArgs &a, double *pc, double *pt, int *nblocks, hipStream_t s);
+hipError_t run_clock_set(int *active, int *target, int *stepc, double *time, int steps, int step, double t,
+                         hipStream_t s);
 hipError_t run_clock(int nslot, const int *run, const double *dt, double *time, int *stepc, int bump, hipStream_t s);
 hipError_t run_sponge(const PassArgs &a, const double *spg, int Mx, int nleft, hipStream_t s);
 // pointwise steps of Compute_hyper and Compute_Grad outside a stage (one

@@ -107,7 +107,7 @@ namespace st {
 template <int NV, class OP>
 DEV void block_reduce(double (&v)[NV], OP op, double *partial, int slot)
 {
-    __shared__ double sh[NV][256 / 64];
+    __shared__ double sh[NV][256 / 64];          // one array per NV: a kernel may reduce 2, then 3 values
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
     for (int i = 0; i < NV; i++) {
@@ -144,31 +144,64 @@ __global__ void __launch_bounds__(256) k_cfl(PassArgs a, double *partial)
     block_reduce<2>(v, OpMax(), partial, slot);
 }
 
+// The three dt limits of Compute_Tstep at a point
+// (src/lddrk4_periodic_sf.f:105-132)
+DEV void limit_point(const Phys &ph, double q1, double q2, double q3, double q4, double q5, double beta, double mu,
+                     double kap, double (&l)[3])
+{
+    const double fac = ph.gamma * ph.gm1;
+    const double del = ph.D[0];
+    const double t1 = 1.0 / q4;
+    const double br = q5 - 0.5 * t1 * (q1 * q1 + q2 * q2 + q3 * q3);
+    const double t2 = sqrt(fac * t1 * br);
+    const double T = ph.gamma * t1 * br;
+    l[0] = q4 * (del * del) / mu;
+    l[1] = q4 * (del * del) / beta;
+    l[2] = q4 * ((del * t2) * (del * t2)) / (kap * T);
+}
+
 // Compute_Tstep src/lddrk4_periodic_sf.f:105-132 (beta*, mu*, kappa* in Hc)
 __global__ void __launch_bounds__(256) k_tstep(PassArgs a, double *partial)
 {
     const int slot = a.slots ? a.slots[blockIdx.y] : blockIdx.y;
     if (a.act && !a.act[slot]) return;
     const long N = a.N, off = (long)slot * a.ni;
-    const Phys &ph = a.ph;
-    const double fac = ph.gamma * ph.gm1;
-    const double del = ph.D[0];
     double v[3] = {INFINITY, INFINITY, INFINITY};
     for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < a.ni; i += (long)gridDim.x * blockDim.x) {
         const long gi = off + i;
-        const double q1 = a.Q[gi], q2 = a.Q[N + gi], q3 = a.Q[2 * N + gi], q4 = a.Q[3 * N + gi], q5 = a.Q[4 * N + gi];
-        const double t1 = 1.0 / q4;
-        const double br = q5 - 0.5 * t1 * (q1 * q1 + q2 * q2 + q3 * q3);
-        const double t2 = sqrt(fac * t1 * br);
-        const double T = ph.gamma * t1 * br;
-        const double w3 = q4 * (del * del) / a.Hc[N + gi];
-        const double w4 = q4 * (del * del) / a.Hc[gi];
-        const double w5 = q4 * ((del * t2) * (del * t2)) / (a.Hc[2 * N + gi] * T);
-        v[0] = w3 < v[0] ? w3 : v[0];
-        v[1] = w4 < v[1] ? w4 : v[1];
-        v[2] = w5 < v[2] ? w5 : v[2];
+        double l[3];
+        limit_point(a.ph, a.Q[gi], a.Q[N + gi], a.Q[2 * N + gi], a.Q[3 * N + gi], a.Q[4 * N + gi], a.Hc[gi],
+                    a.Hc[N + gi], a.Hc[2 * N + gi], l);
+        for (int k = 0; k < 3; k++) v[k] = l[k] < v[k] ? l[k] : v[k];
     }
     block_reduce<3>(v, OpMin(), partial, slot);
+}
+
+// Both in one sweep, for the steps whose dt is formed on the device: Q is
+// read once instead of twice.  The same expressions and the same order within
+// a block as the two above, so the same bits; pt null: no limits (artificial
+// transport off).
+__global__ void __launch_bounds__(256) k_cfl_tstep(PassArgs a, double *pc, double *pt)
+{
+    const int slot = a.slots ? a.slots[blockIdx.y] : blockIdx.y;
+    if (a.act && !a.act[slot]) return;
+    const long N = a.N, off = (long)slot * a.ni;
+    const Phys &ph = a.ph;
+    double v[2] = {-INFINITY, -INFINITY}, u[3] = {INFINITY, INFINITY, INFINITY};
+    for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < a.ni; i += (long)gridDim.x * blockDim.x) {
+        const long gi = off + i;
+        const double q1 = a.Q[gi], q2 = a.Q[N + gi], q3 = a.Q[2 * N + gi], q4 = a.Q[3 * N + gi], q5 = a.Q[4 * N + gi];
+        double w[2];
+        cfl_point(ph, q1, q2, q3, q4, q5, w[0], w[1]);
+        for (int k = 0; k < 2; k++) v[k] = w[k] > v[k] ? w[k] : v[k];
+        if (pt) {
+            double l[3];
+            limit_point(ph, q1, q2, q3, q4, q5, a.Hc[gi], a.Hc[N + gi], a.Hc[2 * N + gi], l);
+            for (int k = 0; k < 3; k++) u[k] = l[k] < u[k] ? l[k] : u[k];
+        }
+    }
+    block_reduce<2>(v, OpMax(), pc, slot);
+    if (pt) block_reduce<3>(u, OpMin(), pt, slot);
 }
 
 // Compute_Mom/KE/Mass/Energy/Entropy src/lddrk4_periodic_sf.f:153-302 (sums)
@@ -222,41 +255,63 @@ __global__ void __launch_bounds__(256) k_fixp(PassArgs a, double *Qx)
     }
 }
 
-// Device-side Compute_Tstep for every slot (one thread per slot): fold the
+// Device-side Compute_Tstep for every slot (one workgroup per slot): fold the
 // CFL and dt-limit partials, dt = cfl_cal/cfl_resv, then the hyper limits
 // when the slot's step passes the driver's rule (src/lddrk4_periodic_sf.f:96-142;
 // first_step = 1 applies them from the first step,
 // src/lddrk4_nonperiodic_sf.f:105).  stepc is the driver's step counter
 // (1 before the first step).  A slot runs this step (run = 1) while it is
-// active and its counter is below its target.
-__global__ void k_dt(const double *pc, const double *pt, int nb, int nslot, const int *active, const int *target,
-                     const int *stepc, double cfl_cal, int hyper, int first_step, int *run, double *dt, double *dt_last)
+// active and its counter is below its target; with hist set, only if its dt is
+// positive and finite, and hist[step - hist0] records the dt.
+// The fold of up to 1024 partials a slot is a chain of dependent loads in one
+// thread (219 us at 64^3); 256 threads take four partials each (5 us).  A
+// maximum or minimum does not depend on the order, NaNs are passed over.
+__global__ void __launch_bounds__(256)
+k_dt(const double *pc, const double *pt, int nb, const int *active, const int *target, const int *stepc, double cfl_cal,
+     int hyper, int first_step, int *run, double *dt, double *dt_last, double *hist, int hist0)
 {
-    const int slot = blockIdx.x * blockDim.x + threadIdx.x;
-    if (slot >= nslot) return;
-    const int go = active[slot] && stepc[slot] < target[slot];
-    run[slot] = go;
-    if (!go) return;
-    double resv = -INFINITY;
-    for (int b = 0; b < nb; b++) {
-        const double x = pc[((long)slot * nb + b) * 2 + 1];
-        resv = x > resv ? x : resv;
+    __shared__ double sh[4][4];
+    const int slot = blockIdx.x;
+    const int step = stepc[slot], go = active[slot] && step < target[slot];
+    if (!go) {                                      // the same on every thread
+        if (threadIdx.x == 0) run[slot] = 0;
+        return;
     }
-    double t = cfl_cal / resv;
-    if (hyper == 1 && (stepc[slot] > 1 || first_step)) {
-        double v[3] = {INFINITY, INFINITY, INFINITY};
-        for (int b = 0; b < nb; b++)
+    const bool lim = hyper == 1 && (step > 1 || first_step);
+    double v[4] = {-INFINITY, INFINITY, INFINITY, INFINITY};
+    for (int b = threadIdx.x; b < nb; b += blockDim.x) {
+        const double x = pc[((long)slot * nb + b) * 2 + 1];
+        v[0] = x > v[0] ? x : v[0];
+        if (lim)
             for (int i = 0; i < 3; i++) {
-                const double x = pt[((long)slot * nb + b) * 3 + i];
-                v[i] = x < v[i] ? x : v[i];
+                const double y = pt[((long)slot * nb + b) * 3 + i];
+                v[1 + i] = y < v[1 + i] ? y : v[1 + i];
             }
+    }
+    for (int i = 0; i < 4; i++) {
+        for (int o = 32; o > 0; o >>= 1) {
+            const double x = __shfl_xor(v[i], o);
+            v[i] = (i == 0 ? x > v[i] : x < v[i]) ? x : v[i];
+        }
+        if ((threadIdx.x & 63) == 0) sh[i][threadIdx.x >> 6] = v[i];
+    }
+    __syncthreads();
+    if (threadIdx.x) return;
+    for (int i = 0; i < 4; i++)
+        for (int w = 1; w < 4; w++) {
+            const double x = sh[i][w];
+            v[i] = (i == 0 ? x > v[i] : x < v[i]) ? x : v[i];
+        }
+    double t = cfl_cal / v[0];
+    if (lim) {
         const double p2 = (double)0.2f;                 // default-real literal 0.2
-        if (p2 * v[0] < t) t = p2 * v[0];
-        if (p2 * v[1] < t) t = p2 * v[1];
-        if (p2 * v[2] < t) t = p2 * v[2];
+        for (int i = 1; i < 4; i++)
+            if (p2 * v[i] < t) t = p2 * v[i];
     }
     dt[slot] = t;
     dt_last[slot] = t;
+    if (hist) hist[step - hist0] = t;
+    run[slot] = !hist || (t > 0.0 && t < INFINITY);
 }
 
 // time += dt after each RK loop; step += 1 after the second
@@ -509,12 +564,36 @@ hipError_t run_fixp(const PassArgs &a, double *Qx, hipStream_t s)
     return hipGetLastError();
 }
 
+hipError_t run_cfl_tstep(const PassArgs &a, double *pc, double *pt, int *nblocks, hipStream_t s)
+{
+    const long nb = red_blocks(a.ni);
+    *nblocks = (int)nb;
+    hipLaunchKernelGGL(k_cfl_tstep, dim3((unsigned)nb, (unsigned)a.nslot), dim3(256), 0, s, a, pc, pt);
+    return hipGetLastError();
+}
+
 hipError_t run_dt(const double *pc, const double *pt, int nb, int nslot, const int *active, const int *target,
                   const int *stepc, double cfl_cal, int hyper, int first_step, int *run, double *dt, double *dt_last,
-                  hipStream_t s)
+                  double *hist, int hist0, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_dt, dim3((unsigned)((nslot + 63) / 64)), dim3(64), 0, s, pc, pt, nb, nslot, active, target,
-                       stepc, cfl_cal, hyper, first_step, run, dt, dt_last);
+    hipLaunchKernelGGL(k_dt, dim3((unsigned)nslot), dim3(256), 0, s, pc, pt, nb, active, target, stepc, cfl_cal, hyper,
+                       first_step, run, dt, dt_last, hist, hist0);
+    return hipGetLastError();
+}
+
+// The clock of one run: active, its target, step and time
+__global__ void k_clock_set(int *active, int *target, int *stepc, double *time, int steps, int step, double t)
+{
+    *active = 1;
+    *target = step + steps;
+    *stepc = step;
+    *time = t;
+}
+
+hipError_t run_clock_set(int *active, int *target, int *stepc, double *time, int steps, int step, double t,
+                         hipStream_t s)
+{
+    hipLaunchKernelGGL(k_clock_set, dim3(1), dim3(1), 0, s, active, target, stepc, time, steps, step, t);
     return hipGetLastError();
 }
 

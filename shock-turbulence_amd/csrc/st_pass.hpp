@@ -570,7 +570,14 @@ struct RaggedArgs {
 };
 static_assert(sizeof(RaggedArgs) <= 4000, "kernel arguments");
 
-template <int NT, class PASS, class F>
+template <int NT, class PASS, class F, int ST>
+DEV void ragged_tile(const Geo &g, const PassArgs &a, long local)
+{
+    if (local >= g.ntiles) return;
+    pass_body<F::M, F::P, NT, false, PASS, ST>(g, a, (ST & STREAM_Y) ? local : tile_of(g, local));
+}
+
+template <int NT, class PASS, class F, int ST>
 __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(PASS::MIN_WAVES)))
 k_ragged(RaggedArgs r)
 {
@@ -580,23 +587,25 @@ k_ragged(RaggedArgs r)
     for (int i = 1; i < RG_MAX; i++) c += wg >= r.start[i] ? 1 : 0;
     const long local = wg - r.start[c];
     switch (c) {
-    case 0:
-        if (local < r.g[0].ntiles)
-            pass_body<F::L0::M, F::L0::P, NT, false, PASS>(r.g[0], r.a[0], tile_of(r.g[0], local));
-        break;
-    case 1:
-        if (local < r.g[1].ntiles)
-            pass_body<F::L1::M, F::L1::P, NT, false, PASS>(r.g[1], r.a[1], tile_of(r.g[1], local));
-        break;
-    case 2:
-        if (local < r.g[2].ntiles)
-            pass_body<F::L2::M, F::L2::P, NT, false, PASS>(r.g[2], r.a[2], tile_of(r.g[2], local));
-        break;
-    default:
-        if (local < r.g[3].ntiles)
-            pass_body<F::L3::M, F::L3::P, NT, false, PASS>(r.g[3], r.a[3], tile_of(r.g[3], local));
-        break;
+    case 0: ragged_tile<NT, PASS, typename F::L0, ST>(r.g[0], r.a[0], local); break;
+    case 1: ragged_tile<NT, PASS, typename F::L1, ST>(r.g[1], r.a[1], local); break;
+    case 2: ragged_tile<NT, PASS, typename F::L2, ST>(r.g[2], r.a[2], local); break;
+    default: ragged_tile<NT, PASS, typename F::L3, ST>(r.g[3], r.a[3], local); break;
     }
+}
+
+template <int NT, class PASS, class F, int ST>
+static hipError_t launch_ragged_s(const RaggedArgs &r, long wg, size_t lds, hipStream_t s)
+{
+    static size_t lds_set = 0;
+    if (lds > 64 * 1024 && lds > lds_set) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_ragged<NT, PASS, F, ST>),
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return e;
+        lds_set = lds;
+    }
+    hipLaunchKernelGGL((k_ragged<NT, PASS, F, ST>), dim3((unsigned)wg), dim3(NT), lds, s, r);
+    return hipGetLastError();
 }
 
 // One ragged launch of PASS: per family member c, the tables t[c] (null:
@@ -607,7 +616,7 @@ static hipError_t launch_ragged(const RaggedSpec &sp, hipStream_t s)
 {
     constexpr int NT = 256;
     RaggedArgs r;
-    long wg = 0;
+    long wg = 0, pts = 0;
     size_t lds = 0;
     for (int c = 0; c < RG_MAX; c++) {
         r.start[c] = wg;
@@ -630,21 +639,20 @@ static hipError_t launch_ragged(const RaggedSpec &sp, hipStream_t s)
         g.tpi = lot / g.B;
         g.ntiles = g.tpi * sp.a[c].nslot;
         wg += (g.ntiles + 7) / 8 * 8;
+        pts += sp.a[c].ni * sp.a[c].nslot;
         const size_t l = (size_t)pass_slots<PASS>() * NT * t.M * sizeof(double);
         lds = l > lds ? l : lds;
     }
     r.start[RG_MAX] = wg;
     if (wg == 0) return hipSuccess;
     if (lds > 160 * 1024) return hipErrorInvalidValue;
-    static size_t lds_set = 0;
-    if (lds > 64 * 1024 && lds > lds_set) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_ragged<NT, PASS, F>),
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return e;
-        lds_set = lds;
+    // (the y passes alone: the family's strided tiles are 8 lines at the larger
+    // sizes)
+    constexpr int ST = stream_n<PASS>::value;
+    if constexpr (ST & STREAM_Y) {
+        if (pts >= STREAM_POINTS) return launch_ragged_s<NT, PASS, F, ST>(r, wg, lds, s);
     }
-    hipLaunchKernelGGL((k_ragged<NT, PASS, F>), dim3((unsigned)wg), dim3(NT), lds, s, r);
-    return hipGetLastError();
+    return launch_ragged_s<NT, PASS, F, 0>(r, wg, lds, s);
 }
 
 }  // namespace st

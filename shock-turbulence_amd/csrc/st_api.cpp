@@ -28,7 +28,7 @@ static_assert(st::K_NPASS <= KIND_RED, "pass kinds overlap the other timed kinds
 const char *kind_names[NKIND] = {
     "d1", "d2", "filter", "gauss", "grad", "lap_se",
     "lap2", "lap2_gauss", "gauss_eta", "gauss_hdiv", "hyper_div", "rk_filter", "filter_q",
-    "filter_q_fix", "grad_cross", "hdiv_rkf", "lap_se_lap2", "", "", "", "", "reduce", "fill", ""};
+    "filter_q_fix", "grad_cross", "hdiv_rkf", "lap_se_lap2", "fq_grad", "", "", "", "reduce", "fill", ""};
 
 struct Event {
     hipEvent_t a, b;
@@ -188,7 +188,7 @@ double kind_fields(int kind, int dir, const st::PassArgs &a)
     // Q, G of the direction, the dQ partial, the Lap e partial; z also reads
     // the two stored derivatives of its mixed terms
     case st::K_GRAD: return 5 + 4 + 5 + (a.L2e ? 1 : 0) + (dir == 2 ? 2 : 0);
-    case st::K_LAPSE: return a.first ? 2 + 2 : 2 + 4;
+    case st::K_LAPSE: return 2 + 4;
     case st::K_LAP2: return a.first ? 2 : 3;
     // L2S, L4S, L4e, Q in; eta out
     case st::K_LAP2_LAST: return 1 + 1 + 1 + 5 + 2;
@@ -208,8 +208,10 @@ double kind_fields(int kind, int dir, const st::PassArgs &a)
     // Q, G of y (written), 8 G of x and z (the four inputs of the mixed
     // terms and four more), the z and x partials, dQ (written); with the
     // artificial transport the Laplacian of e (2 partials in, the sum out),
-    // |S| and C_beta
-    case st::K_GRAD_CROSS: return 5 + 4 + 8 + 10 + 5 + (a.L2e ? 3 + 1 + (a.Cb ? 1 : 0) : 0);
+    // |S|, C_beta and the y terms of two Laplacians
+    case st::K_GRAD_CROSS: return 5 + 4 + 8 + 10 + 5 + (a.L2e ? 3 + 1 + (a.Cb ? 1 : 0) + 2 : 0);
+    // Q (read and written), then as grad x
+    case st::K_FQ_GRAD: return 10 + 4 + 5 + (a.L2e ? 1 : 0);
     default: return 0;
     }
 }
@@ -698,10 +700,21 @@ int fill(st_ctx *c, double *p, int nfields, const st::PassArgs &base, double v)
     return 0;
 }
 
+// The arguments of the x gradient pass: its own partial sums.
+st::PassArgs grad_x_args(st_ctx *c, const st::PassArgs &base)
+{
+    st::PassArgs b = base;
+    b.first = 1;
+    b.dQ = c->dQp + 5 * c->N;
+    b.L2e = c->p.hyper_param ? c->L2ep + c->N : nullptr;
+    return b;
+}
+
 // RHS (src/rhsv_periodic_sf.f:9-25) into dQ; with the artificial transport
-// on, also the strain magnitude, the sensor and the x and y parts of the
-// first Laplacians it needs.
-int seq_rhs(st_ctx *c, const st::PassArgs &base)
+// on, also the strain magnitude, the sensor and the y and x parts of the
+// first Laplacians it needs.  have_x: the x pass has been done (by the last
+// pass of the stage before).
+int seq_rhs(st_ctx *c, const st::PassArgs &base, bool have_x = false)
 {
     const int hyp = c->p.hyper_param;
     st::PassArgs a = base;
@@ -710,23 +723,17 @@ int seq_rhs(st_ctx *c, const st::PassArgs &base)
     // the y pass adds them up with its own terms and the viscous products.
     // z and y also take the mixed second derivatives, from the x (and z)
     // derivatives stored before them.
+    if (!have_x) TRY(pass(c, st::K_GRAD, 0, grad_x_args(c, base)));
     {
         st::PassArgs b = a;
-        b.dQ = c->dQp + 5 * c->N;
-        b.L2e = hyp ? c->L2ep + c->N : nullptr;
-        TRY(pass(c, st::K_GRAD, 0, b));
         b.dQ = c->dQp;
         b.L2e = hyp ? c->L2ep : nullptr;
         TRY(pass(c, st::K_GRAD, 2, b));
     }
     TRY(pass(c, st::K_GRAD_CROSS, 1, a));
-    if (hyp) {
-        // D2 of |S| and Lap e, summed over x, y (z joins the first pass of
-        // the artificial transport)
-        TRY(pass(c, st::K_LAPSE, 0, a));
-        a.first = 0;
-        TRY(pass(c, st::K_LAPSE, 1, a));
-    }
+    // D2 of |S| and Lap e: y in the pass before, x here (z joins the first
+    // pass of the artificial transport)
+    if (hyp) TRY(pass(c, st::K_LAPSE, 0, a));
     return 0;
 }
 
@@ -753,12 +760,14 @@ int seq_hyper(st_ctx *c, const st::PassArgs &base, const st::PassArgs *rk = null
     return 0;
 }
 
-// One stage body (src/lddrk4_periodic_sf.f:344-356).  last: the coefficients
-// /HYPER/ are left in Hc (the stages before the last of a step rewrite them
-// before anything reads them).  guard: a run flag for the passes that write
-// the state alone (the others then start without waiting for a flag).
-int seq_stage(st_ctx *c, const st::PassArgs &base0, double ra, double rb, double dt, bool last = true,
-              const int *guard = nullptr)
+// One stage body (src/lddrk4_periodic_sf.f:344-356).  A stage of a step that
+// is not its first (have_x) or not its last (!last) shares the x pass between
+// them with its neighbour.  last: the coefficients /HYPER/ are left in Hc (the
+// stages before the last of a step rewrite them before anything reads them).
+// guard: a run flag for the passes that write the state alone (the others
+// then start without waiting for a flag).
+int seq_stage(st_ctx *c, const st::PassArgs &base0, double ra, double rb, double dt, bool have_x = false,
+              bool last = true, const int *guard = nullptr)
 {
     st::PassArgs base = base0;
     base.keep_hc = last ? 1 : 0;
@@ -767,10 +776,15 @@ int seq_stage(st_ctx *c, const st::PassArgs &base0, double ra, double rb, double
     a.rk_a = ra;
     a.rk_b = rb;
     a.dt = dt;
-    TRY(seq_rhs(c, base));
+    const bool sep = getenv("ST_NO_FUSE_RK") != nullptr;
+    // (the closure rows and corrections of both halves cost a large
+    // non-periodic grid more registers than the fusion saves memory time:
+    // 512 x 192 x 192, 1703 us fused against 948 + 607)
+    const bool share = !sep && !(c->g.nonperiodic_x && c->ni >= st::STREAM_POINTS);
+    TRY(seq_rhs(c, base, have_x && share));
     // the update (and the sponge term before it) joins the last divergence
     // pass
-    const bool fuse = c->p.hyper_param && !getenv("ST_NO_FUSE_RK");
+    const bool fuse = c->p.hyper_param && !sep;
     if (fuse && c->spg) {
         a.spg = c->spg;
         a.spg_left = c->spg_left;
@@ -780,10 +794,12 @@ int seq_stage(st_ctx *c, const st::PassArgs &base0, double ra, double rb, double
         const hipError_t e = st::run_sponge(base, c->spg, c->Mx, c->spg_left, c->s);
         if (e != hipSuccess) return fail(c, -4, "sponge: %s", hipGetErrorString(e));
     }
-    // filters y (with the update), z, x (with Fix_Pressure)
+    // filters y (with the update), z, x (with Fix_Pressure, and the x gradient
+    // pass of the next stage)
     if (!fuse) TRY(pass(c, st::K_RKF, 1, a));
     TRY(pass(c, st::K_FQ, 2, a));
     a.fix = 1;
+    if (!last && share) return pass(c, st::K_FQ_GRAD, 0, grad_x_args(c, a));
     TRY(pass(c, st::K_FQ_FIX, 0, a));
     return 0;
 }
@@ -899,7 +915,7 @@ int stage_loop(st_ctx *c, double dt, double *time, int *step)
         if (!ns) break;
         // QW = 0 at the loop start (:339, :376): the first stage's alpha is 0
         // and the update then does not read QW
-        for (int k = 0; k < ns; k++) TRY(seq_stage(c, base, ra[k], rb[k], dt, last_stage(c->p.rk_scheme, loop, k)));
+        for (int k = 0; k < ns; k++) TRY(seq_stage(c, base, ra[k], rb[k], dt, loop || k, last_stage(c->p.rk_scheme, loop, k)));
         if (time) *time = *time + dt;                        // :372, :419
     }
     if (step) *step = *step + 1;                             // :420
@@ -932,7 +948,7 @@ int batch_step(st_ctx *c)
         const int ns = rk_loop(c->p.rk_scheme, loop, &ra, &rb);
         if (!ns) break;
         for (int k = 0; k < ns; k++)                         // (QW: as stage_loop)
-            TRY(seq_stage(c, a, ra[k], rb[k], 0.0, last_stage(c->p.rk_scheme, loop, k)));
+            TRY(seq_stage(c, a, ra[k], rb[k], 0.0, loop || k, last_stage(c->p.rk_scheme, loop, k)));
         const int last = loop == 1 || !rk_loop(c->p.rk_scheme, 1, &ra, &rb);
         err = st::run_clock(c->ns, c->s_run, c->s_dt, c->s_time, c->s_step, last, c->s);
         if (err != hipSuccess) return fail(c, -4, "batch clock: %s", hipGetErrorString(err));
@@ -1211,7 +1227,7 @@ extern "C" int st_march(st_ctx *c, int nsteps, double *time, int *step, double *
                 const int ns = rk_loop(c->p.rk_scheme, loop, &ra, &rb);
                 if (!ns) break;
                 for (int k = 0; k < ns; k++)                 // (QW: as stage_loop)
-                    TRY(seq_stage(c, a, ra[k], rb[k], 0.0, last_stage(c->p.rk_scheme, loop, k), run));
+                    TRY(seq_stage(c, a, ra[k], rb[k], 0.0, loop || k, last_stage(c->p.rk_scheme, loop, k), run));
                 err = st::run_clock(1, run, dt, tm, stepc, last_stage(c->p.rk_scheme, loop, ns - 1), c->s);
                 if (err != hipSuccess) return fail(c, -4, "march clock: %s", hipGetErrorString(err));
             }
@@ -1363,12 +1379,13 @@ namespace {
 
 // Record one stage of member m (nothing is launched); the member's passes
 // all take the M/2-point layouts of the size family.
-int group_record(st_ctx *m, const st::PassArgs &a, double ra, double rb, bool last, std::vector<Rec> &out)
+int group_record(st_ctx *m, const st::PassArgs &a, double ra, double rb, bool have_x, bool last,
+                 std::vector<Rec> &out)
 {
     out.clear();
     m->rec = &out;
     m->force_narrow = 1;
-    const int r = seq_stage(m, a, ra, rb, 0.0, last);
+    const int r = seq_stage(m, a, ra, rb, 0.0, have_x, last);
     m->rec = nullptr;
     m->force_narrow = 0;
     return r;
@@ -1413,7 +1430,8 @@ int group_step(st_group *G)
             for (int c = c0; c < 4; c++) {
                 st_ctx *m = G->m[c];
                 if (!m || !m->nact) continue;
-                if (group_record(m, a[c], ra[k], rb[k], last_stage(p.rk_scheme, loop, k), rec[c]))
+                if (group_record(m, a[c], ra[k], rb[k], loop || k, last_stage(p.rk_scheme, loop, k),
+                                 rec[c]))
                     return st::set_call_error(-4, "group stage (%d points): %s", m->Mx, m->err);
                 if (rec[c].size() != rec[c0].size())
                     return st::set_call_error(-4, "group stage: members record different pass sequences");
@@ -1639,7 +1657,11 @@ extern "C" int st_autotune(st_ctx *c, int reps)
         c->prof = 1;
         std::memset(c->prof_ms, 0, sizeof(c->prof_ms));
         std::memset(c->prof_cnt, 0, sizeof(c->prof_cnt));
-        for (int r = 0; r < reps && !rc; r++) rc = seq_stage(c, base, ra[0], rb[0], 1.0e-6);
+        for (int r = 0; r < reps && !rc; r++) {
+            // two stages of a step, so that every pass of one is timed
+            rc = seq_stage(c, base, ra[0], rb[0], 1.0e-6, false, false);
+            if (!rc) rc = seq_stage(c, base, ra[1], rb[1], 1.0e-6, true, true);
+        }
         if (hipStreamSynchronize(c->s) != hipSuccess && !rc) rc = fail(c, -3, "autotune: stream error");
         prof_collect(c);
         for (int k = st::K_GRAD; k < st::K_NPASS; k++)

@@ -76,6 +76,7 @@ enum PassKind {
     K_GRAD_CROSS,
     K_HDIV_RKF,
     K_LAPSE_LAP2,
+    K_FQ_GRAD,
     K_NPASS,              // pass kinds end here
 };
 
@@ -103,6 +104,7 @@ hipError_t run_pass_ragged(int kind, const RaggedSpec &sp, hipStream_t s);
 hipError_t launch_grad_x_ragged(const RaggedSpec &sp, hipStream_t s);
 hipError_t launch_grad_y_ragged(const RaggedSpec &sp, hipStream_t s);
 hipError_t launch_grad_z_ragged(const RaggedSpec &sp, hipStream_t s);
+hipError_t launch_fqgrad_ragged(const RaggedSpec &sp, hipStream_t s);
 hipError_t launch_lapse_ragged(int kind, const RaggedSpec &sp, hipStream_t s);
 hipError_t launch_hyper_ragged(int kind, const RaggedSpec &sp, hipStream_t s);
 hipError_t launch_hdivrk_ragged(int kind, const RaggedSpec &sp, hipStream_t s);
@@ -126,6 +128,7 @@ hipError_t run_pass(int kind, const DirTab &t, int nt, int dir, int My, int Mz, 
 // per translation unit (st_pass_*.hip)
 hipError_t launch_ops(int kind, const DirTab &t, int nt, int dir, int My, int Mz, int Mx, const PassArgs &a, hipStream_t s);
 hipError_t launch_grad_x(const DirTab &t, int nt, int My, int Mz, int Mx, const PassArgs &a, hipStream_t s);
+hipError_t launch_fqgrad(const DirTab &t, int nt, int My, int Mz, int Mx, const PassArgs &a, hipStream_t s);
 hipError_t launch_grad_y(const DirTab &t, int nt, int My, int Mz, int Mx, const PassArgs &a, hipStream_t s);
 hipError_t launch_grad_z(const DirTab &t, int nt, int My, int Mz, int Mx, const PassArgs &a, hipStream_t s);
 hipError_t launch_lapse(int kind, const DirTab &t, int nt, int dir, int My, int Mz, int Mx, const PassArgs &a, hipStream_t s);

@@ -62,6 +62,8 @@ hipError_t run_pass(int kind, const DirTab &t, int nt, int dir, int My, int Mz, 
         return launch_hyper(kind, t, nt, dir, My, Mz, Mx, a, s);
     case K_RKF: case K_FQ: case K_FQ_FIX:
         return launch_filter(kind, t, nt, dir, My, Mz, Mx, a, s);
+    case K_FQ_GRAD:
+        return dir == 0 ? launch_fqgrad(t, nt, My, Mz, Mx, a, s) : hipErrorInvalidValue;
     case K_HDIV_RKF:
         return launch_hdivrk(kind, t, nt, dir, My, Mz, Mx, a, s);
     default: return hipErrorInvalidValue;
@@ -90,6 +92,8 @@ hipError_t run_pass_ragged(int kind, const RaggedSpec &sp, hipStream_t s)
         return launch_hyper_ragged(kind, sp, s);
     case K_RKF: case K_FQ: case K_FQ_FIX:
         return launch_filter_ragged(kind, sp, s);
+    case K_FQ_GRAD:
+        return sp.dir == 0 ? launch_fqgrad_ragged(sp, s) : hipErrorInvalidValue;
     case K_HDIV_RKF:
         return launch_hdivrk_ragged(kind, sp, s);
     default: return hipErrorInvalidValue;

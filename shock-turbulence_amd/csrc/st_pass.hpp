@@ -80,7 +80,7 @@ struct carry_n<T, std::void_t<decltype(T::NCARRY)>> { static constexpr int value
 // compute(), mid() rewrites the NSLOT staged values of each point in memory
 // order (it may read and write global fields of its own points; it also gets
 // the point's index along the line), then compute2() runs on the rewritten
-// slots in the line mapping.
+// slots in the line mapping and leaves the NOUT register results (if any).
 // NKEEP of a pass (0 when it names none): the last NKEEP staged input
 // slots, which compute() only reads, are handed to store() after the late
 // results, so the store phase need not read those fields again.
@@ -153,6 +153,15 @@ template <class T, class = void>
 struct stream_n { static constexpr int value = 0; };
 template <class T>
 struct stream_n<T, std::void_t<decltype(T::STREAM)>> { static constexpr int value = T::STREAM; };
+
+// NPOST of a pass (0 when it names none): values per point that its late
+// store leaves in slots 0..NPOST-1 for a last compute phase on the same lines,
+// compute_post(), whose results store_post() writes; all of it only if
+// post_on(a) (the same on every thread).
+template <class T, class = void>
+struct post_n { static constexpr int value = 0; };
+template <class T>
+struct post_n<T, std::void_t<decltype(T::NPOST)>> { static constexpr int value = T::NPOST; };
 
 template <class T, class = void>
 struct has_mid { static constexpr bool value = false; };
@@ -248,7 +257,7 @@ DEV void pass_body(const Geo &g, const PassArgs &a0, long tile)
     asm volatile("" : "+v"(tl));
     const Walk<M, P, NT> Wl(g, tile - (long)si * g.tpi, (long)slot * a.ni, tl);
     if constexpr (has_mid<PASS>::value) {
-        static_assert(RE && NO == 0, "a second compute phase works on the slots");
+        static_assert(RE, "a second compute phase works on the slots");
         constexpr int NMF = mf_n<PASS>::value, MFB = mf_n<PASS>::batch < M ? mf_n<PASS>::batch : M;
         __syncthreads();
 #pragma unroll
@@ -278,7 +287,8 @@ DEV void pass_body(const Geo &g, const PassArgs &a0, long tile)
             }
         }
         __syncthreads();
-        PASS::template compute2<M, P, NP>(g, a, L);
+        if constexpr (NO > 0) PASS::template compute2<M, P, NP>(g, a, L, out);
+        else PASS::template compute2<M, P, NP>(g, a, L);
     }
 
     // 3. store (through LDS, memory order)
@@ -354,10 +364,35 @@ DEV void pass_body(const Geo &g, const PassArgs &a0, long tile)
 #pragma unroll
             for (int q = 0; q < NPF; q++) v[NV + NK + q] = pf[r][q];
             static_assert(NLC == 0 || (NSF > 0 && NCR > 0), "a load carry to the store goes with store-phase fetches and a carry");
-            if constexpr (NLC > 0) PASS::store(g, a, gi, v, cr[r], sf[j], lc[r]);
+            constexpr int NPO = post_n<PASS>::value;
+            static_assert(NPO == 0 || (RE && NLC > 0 && NPO <= NO), "values for the last phase take the late results' slots");
+            if constexpr (NPO > 0) {
+                double po[NPO];
+                PASS::store(g, a, gi, v, cr[r], sf[j], lc[r], po);
+#pragma unroll
+                for (int q = 0; q < NPO; q++) lds[q * ss + li] = po[q];
+            } else if constexpr (NLC > 0) PASS::store(g, a, gi, v, cr[r], sf[j], lc[r]);
             else if constexpr (NSF > 0) PASS::store(g, a, gi, v, cr[r], sf[j]);
             else if constexpr (NCR > 0) PASS::store(g, a, gi, v, cr[r]);
             else PASS::store(g, a, gi, v);
+        }
+    }
+
+    // 4. last phase
+    if constexpr (post_n<PASS>::value > 0) {
+        if (!PASS::post_on(a)) return;
+        __syncthreads();
+        PASS::template compute_post<M, P, NP>(a, L);
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < M; r++) {
+            int b, s;
+            const long gi = Wl.at(g, r, b, s);
+            const int li = lds_idx<M, AL>(b, s % M, s / M, P, lds_g<M>(b, NT / P));
+            double v[post_n<PASS>::value];
+#pragma unroll
+            for (int q = 0; q < post_n<PASS>::value; q++) v[q] = lds[q * ss + li];
+            PASS::store_post(a, gi, v);
         }
     }
 }

@@ -62,7 +62,12 @@ struct PassGrad {
     static constexpr int NLCARRY = CROSS ? 4 : 0;
     HD static constexpr int hold_slot(int j) { return j == 0 ? 1 : 4; }
     static constexpr bool REUSE = true;
-    static constexpr int NCARRY = CROSS ? 4 : 0;
+    // (CROSS: the y derivatives and the Laplacian of e)
+    static constexpr int NCARRY = CROSS ? 5 : 0;
+    // CROSS: |S| and the Laplacian of e, complete here, are differentiated
+    // twice along y while their lines are at hand (the first terms of Lap|S|
+    // and Lap(Lap e)): a pass less, two fields fewer
+    static constexpr int NPOST = CROSS ? 2 : 0;
     // CROSS: the staged inputs of the mixed terms (du/dx, dv/dx, dv/dz,
     // dw/dz) and the viscosity reach the store after the late results
     static constexpr int NKEEP = CROSS ? NMX + 1 : 0;
@@ -351,7 +356,8 @@ struct PassGrad {
         a.G[10 * N + gi] = v[3];
 #pragma unroll
         for (int c = 0; c < 4; c++) cr[c] = v[c];
-        if (a.L2e) a.L2e[gi] = (v[4] + sf[0]) + sf[1];
+        cr[4] = (v[4] + sf[0]) + sf[1];
+        if (a.L2e) a.L2e[gi] = cr[4];
     }
     // the store phase's reads: du/dz, dw/dx, dT/dx, dT/dz, the z partials
     // (5), the x partials (5)
@@ -375,7 +381,7 @@ struct PassGrad {
     // the artificial transport on (L2e set).
     template <class A>
     DEV static void store(const Geo &, const A &a, long gi, const double *v, const double *cr,
-                          const double *sf, const double *lc)
+                          const double *sf, const double *lc, double *po)
     {
         const long N = a.N;
         const Phys &ph = a.ph;
@@ -403,9 +409,12 @@ struct PassGrad {
                               + mu * (2.0 * (gxx * gxx + gyy * gyy + gzz * gzz) + f1 * dil * dil)
                               + mu * (t1 * t1 + t2 * t2 + t3 * t3)
                               + ph.pr_inv * (ty * cr[3]));
+        po[0] = 0.0;
+        po[1] = cr[4];
         if (a.L2e) {
             const double s12 = 0.5 * (gxy + gyx), s13 = 0.5 * (gxz + gzx), s23 = 0.5 * (gyz + gzy);
-            a.S[gi] = sqrt(0.5 * (gxx * gxx + gyy * gyy + gzz * gzz + 2.0 * (s12 * s12 + s13 * s13 + s23 * s23)));
+            po[0] = sqrt(0.5 * (gxx * gxx + gyy * gyy + gzz * gzz + 2.0 * (s12 * s12 + s13 * s13 + s23 * s23)));
+            a.S[gi] = po[0];
             if (a.Cb) {
                 const double wx = gzy - gyz, wy = gxz - gzx, wz = gyx - gxy;
                 const double om2 = wx * wx + wy * wy + wz * wz;
@@ -413,6 +422,29 @@ struct PassGrad {
                 a.Cb[gi] = fac * dil * dil / (dil * dil + om2 + 1.0e-7) + 1.0e-20;
             }
         }
+    }
+    // CROSS: D2y of |S| and Lap e
+    template <class A>
+    DEV static bool post_on(const A &a) { return (bool)a.L2e; }
+    template <int M, int P, bool NP, bool AL, class A>
+    DEV static void compute_post(const A &a, const Lane<M, P, NP, AL> &L)
+    {
+#pragma unroll 1
+        for (int m = 0; m < 2; m++) {
+            double f[M], w[M + 2 * d_halo<NP>()], r[M];
+#pragma unroll
+            for (int k = 0; k < M; k++) f[k] = L.ld(m, k);
+            window<M>(f, L, w);
+            op_d2<M>(w, a.K2, a.tab()->op[1], L, r);
+#pragma unroll
+            for (int k = 0; k < M; k++) L.st(m, k, r[k]);
+        }
+    }
+    template <class A>
+    DEV static void store_post(const A &a, long gi, const double *v)
+    {
+        a.L2S[gi] = v[0];
+        a.L4e[gi] = v[1];
     }
 };
 

@@ -1,31 +1,26 @@
 // Second derivatives of |S| and of the Laplacian of e (the artificial
-// transport's fourth-order drivers).
+// transport's fourth-order drivers), x.
 #include "st_pass.hpp"
 
 namespace st {
 
 // ---------------------------------------------------------------------
-// D2 along the sweep of |S| and of Lap e, summed over the three directions
-// into L2S = Lap|S| and L4e = Lap(Lap e) (src/hyper_dynamic.f:272-276).
-// ACC = false overwrites (the first direction), true adds to the sums of
-// the earlier directions (prefetched).  The mixed second derivatives of the
-// viscous terms are done in the z and y first-derivative passes.
+// D2 along x of |S| and of Lap e, added to the y terms that the y gradient
+// pass left in L2S = Lap|S| and L4e = Lap(Lap e) (src/hyper_dynamic.f:
+// 272-276); z joins the first pass of the artificial transport.
 // ---------------------------------------------------------------------
-template <bool ACC>
 struct PassLapSE {
-    static constexpr int STREAM = ACC ? STREAM_LOADS | STREAM_Y : STREAM_LOADS;
+    static constexpr int STREAM = STREAM_LOADS;
     static constexpr int NSLOT = 2, NOUT = 0, NEARLY = 2;
     static constexpr bool REUSE = true;
     static constexpr int MIN_WAVES = 1;
     static constexpr int LOAD_UNROLL = 8;
-    static constexpr int NPF = ACC ? 2 : 0;
+    static constexpr int NPF = 2;
     template <class A>
     DEV static void prefetch(const Geo &, const A &a, long gi, double *p)
     {
-        if (ACC) {
-            p[0] = a.L2S[gi];
-            p[1] = a.L4e[gi];
-        }
+        p[0] = a.L2S[gi];
+        p[1] = a.L4e[gi];
     }
     template <class A>
     DEV static void load(const Geo &, const A &a, long gi, double (&v)[2])
@@ -52,13 +47,8 @@ struct PassLapSE {
     template <class A>
     DEV static void store_early(const Geo &, const A &a, long gi, const double *v)
     {
-        if constexpr (ACC) {
-            a.L2S[gi] = v[2] + v[0];
-            a.L4e[gi] = v[3] + v[1];
-        } else {
-            a.L2S[gi] = v[0];
-            a.L4e[gi] = v[1];
-        }
+        a.L2S[gi] = v[2] + v[0];
+        a.L4e[gi] = v[3] + v[1];
     }
 };
 
@@ -66,15 +56,13 @@ struct PassLapSE {
 hipError_t launch_lapse(int kind, const DirTab &t, int nt, int dir, int My, int Mz, int Mx, const PassArgs &a, hipStream_t s)
 {
     if (kind != K_LAPSE) return hipErrorInvalidValue;
-    if (a.first) return launch<PassLapSE<false>>(t, nt, dir, My, Mz, Mx, a, s);
-    return launch<PassLapSE<true>>(t, nt, dir, My, Mz, Mx, a, s);
+    return launch<PassLapSE>(t, nt, dir, My, Mz, Mx, a, s);
 }
 
 hipError_t launch_lapse_ragged(int kind, const RaggedSpec &sp, hipStream_t s)
 {
     if (kind != K_LAPSE) return hipErrorInvalidValue;
-    if (sp.a[sp.first].first) return launch_ragged<PassLapSE<false>>(sp, s);
-    return launch_ragged<PassLapSE<true>>(sp, s);
+    return launch_ragged<PassLapSE>(sp, s);
 }
 
 }  // namespace st

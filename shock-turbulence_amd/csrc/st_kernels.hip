@@ -16,31 +16,41 @@ namespace st {
 
 // Launch shape of a pass: the lane layout (wide: M points per lane on P lanes;
 // narrow: M/2 on 2P) and the threads per workgroup.  Measured with each pass
-// varied in turn and the whole stage timed (us per stage, old -> new shapes).
+// varied in turn and the whole stage timed (us per stage).
 // Grids below STREAM_POINTS live in the caches and launch few workgroups: the
 // narrow layout halves each lane's serial work and 256-thread tiles give the
-// most workgroups (64^3 190 -> 153, 48^3 149 -> 117, 32^3 113 -> 88, 96^3 410
-// -> 353).  Larger grids are bound by memory: unit-stride (y) passes keep the
-// narrow layout and 256 threads; strided passes take the layout of 32 lanes
-// per line and tiles of 16 lines, whose rows are whole 128-byte lines that can
-// stream (256^3: x gradient 5579 -> 5465, z Gaussian and divergence 5476 ->
-// 5405); but for the passes with much arithmetic per point, the z gradient
-// (its two-round form where it exists, else narrow) and the filters, 256
-// threads, more than one workgroup per CU, do better (256^3 filter z 5382
-// against 5447).  The layout decides the rounding, so it depends on the
-// instance alone and not on how many share the launch.
+// most workgroups (against the shapes of 256^3: 64^3 190 -> 153, 48^3 149 ->
+// 117, 32^3 113 -> 88, 96^3 410 -> 353).
+// Larger grids are bound by memory.  y passes keep the narrow layout and 256
+// threads (the plain update and filter 512: 128^3 without artificial transport
+// 393 -> 387).  Strided passes take tiles of 16 lines, whose rows are whole
+// 128-byte lines that can stream (256^3: x gradient 5579 -> 5465, z Gaussian and
+// divergence 5476 -> 5405), on 32 lanes per line (128^3: z Gaussian and
+// divergence narrow 737, wide 751); but the x filter and x gradient passes and
+// their fused form keep the wide layout (128^3: fused 713 wide, 730 narrow),
+// and the filters alone, with much arithmetic for ten fields, 256 threads, more
+// than one workgroup per CU (256^3 filter z 5382 against 5447).  The layout
+// decides the rounding, so it depends on the instance alone and not on how
+// many share the launch.
 void pass_default_cfg(int kind, int dir, const DirTab &wide, long ni, long N, int *narrow, int *nt)
 {
     *narrow = 1;
     *nt = 256;
-    const bool split = wide.M % 2 == 0 && 2 * wide.P <= 64;       // a narrow layout exists
-    const bool compute = kind == K_FQ || kind == K_FQ_FIX || kind == K_GRAD;
-    if (dir != 1 && ni >= STREAM_POINTS) {
-        *narrow = kind == K_GRAD && dir == 2 ? !(wide.M == 8 && wide.P == 32) : wide.P < 32;
-        if (kind == K_D1 || kind == K_D2 || kind == K_FILT || kind == K_GAUSS) *narrow = 0;
+    const bool big = ni >= STREAM_POINTS, many = N >= STREAM_POINTS;
+    if (dir == 1) {
+        if (kind == K_RKF && many) *nt = 512;
+        return;
     }
-    const int P = *narrow && split ? 2 * wide.P : wide.P;
-    if (dir != 1 && N >= STREAM_POINTS && !(compute && !(kind == K_GRAD && dir == 0))) *nt = P <= 16 ? 256 : P == 32 ? 512 : 1024;
+    const bool filt = kind == K_FQ || kind == K_FQ_FIX, xgrad = kind == K_FQ_GRAD || (kind == K_GRAD && dir == 0);
+    if (big) *narrow = !(filt || xgrad) && wide.P < 32;
+    if (many && !filt) {
+        const bool split = wide.M % 2 == 0 && 2 * wide.P <= 64;       // a narrow layout exists
+        const int P = *narrow && split ? 2 * wide.P : wide.P;
+        const int M = *narrow && split ? wide.M / 2 : wide.M;
+        *nt = P <= 16 ? 256 : P == 32 ? 512 : 1024;
+        // the z gradient pass has its 512-thread form for 4 to 7 points per lane
+        if (kind == K_GRAD && dir == 2 && !(P == 32 && M >= 4 && M <= 7)) *nt = 256;
+    }
 }
 
 hipError_t run_pass(int kind, const DirTab &t, int nt, int dir, int My, int Mz, int Mx, const PassArgs &a, hipStream_t s)

@@ -72,7 +72,7 @@ struct PassGrad {
     // dw/dz) and the viscosity reach the store after the late results
     static constexpr int NKEEP = CROSS ? NMX + 1 : 0;
     static constexpr int MIN_WAVES = MW;
-    static constexpr int STREAM = DIR == 2 ? 0 : STREAM_LOADS | STREAM_STORES | (DIR == 1 ? STREAM_Y : 0);
+    static constexpr int STREAM = DIR == 2 && !TWO ? 0 : STREAM_LOADS | STREAM_STORES | (DIR == 1 ? STREAM_Y : 0);
     static constexpr int LOAD_UNROLL = 8;
     static constexpr int NPF = 0;
     // the additive LDS layout for the x and y sweeps (fewer address
@@ -80,7 +80,7 @@ struct PassGrad {
     // pass runs 2% faster) and for z at 8 points per lane; the swizzled one
     // for z at 4 points per lane, whose 4-line tiles would take 4-way bank
     // conflicts in the staging
-    HD static constexpr bool lds_add(int m) { return NMX != 2 || m >= 8; }
+    HD static constexpr bool lds_add(int m) { return NMX != 2 || m >= 8 || TWO; }
     // CROSS: the store phases' global reads (sfetch_early: the z and x
     // partials of the Laplacian of e; sfetch: four x and z derivatives, and
     // the z and x partial sums) go out for all the thread's points (two at a

@@ -1,15 +1,20 @@
 // Host side of the C-ABI (include/st_api.h): context, buffers, pass
 // sequencing for RHS / Hyper_RHS / LDDRK4, reductions and profiling.
 #include <hip/hip_runtime.h>
-#include <omp.h>
 
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
 #include <array>
+#include <atomic>
+#include <condition_variable>
 #include <cstring>
+#include <exception>
 #include <map>
+#include <mutex>
+#include <new>
+#include <thread>
 #include <vector>
 
 #include "../../include/st_api.h"
@@ -33,6 +38,86 @@ const char *kind_names[NKIND] = {
 struct Event {
     hipEvent_t a, b;
     int kind;             // pass kind * 3 + direction
+};
+
+// The helper threads of a context's host transfers, made at its first large
+// one and joined with it.  Between transfers they sleep; within one they share
+// each piece with the calling thread and poll for the next (a piece is some
+// tens of microseconds).  Threads that cannot be had are done without.
+class Copiers {
+public:
+    Copiers()
+    {
+        const int hw = (int)std::thread::hardware_concurrency();
+        const int n = hw - 1 < 0 ? 0 : hw - 1 < MOST ? hw - 1 : MOST;
+        try {
+            for (; have < n; have++) t[have] = std::thread([this, k = have] { work(k + 1); });
+        } catch (const std::exception &) {
+        }
+    }
+    ~Copiers()
+    {
+        set(&stop, true);
+        for (int k = 0; k < have; k++) t[k].join();
+    }
+    Copiers(const Copiers &) = delete;
+    Copiers &operator=(const Copiers &) = delete;
+    void begin() { set(&awake, true); }
+    void end() { set(&awake, false); }
+    // between begin() and end()
+    void copy(void *d, const void *s, size_t n)
+    {
+        dst = (char *)d;
+        src = (const char *)s;
+        size = n;
+        left.store(have, std::memory_order_relaxed);
+        turn.fetch_add(1, std::memory_order_release);
+        part(0);
+        while (left.load(std::memory_order_acquire) > 0) std::this_thread::yield();
+    }
+
+private:
+    static constexpr int MOST = 4;
+    void set(std::atomic<bool> *flag, bool v)
+    {
+        {
+            std::lock_guard<std::mutex> l(mu);
+            flag->store(v);
+        }
+        if (v) cv.notify_all();
+    }
+    void part(int k) const
+    {
+        const size_t each = (size / (have + 1) + 63) & ~(size_t)63, o = each * k;
+        if (o < size) std::memcpy(dst + o, src + o, size - o < each || k == have ? size - o : each);
+    }
+    void work(int k)
+    {
+        for (long seen = 0;;) {
+            if (turn.load(std::memory_order_acquire) != seen) {
+                seen++;
+                part(k);
+                left.fetch_sub(1, std::memory_order_release);
+            } else if (stop) {
+                return;
+            } else if (awake) {
+                std::this_thread::yield();
+            } else {
+                std::unique_lock<std::mutex> l(mu);
+                cv.wait(l, [this] { return stop || awake; });
+            }
+        }
+    }
+    std::thread t[MOST];
+    int have = 0;
+    char *dst = nullptr;
+    const char *src = nullptr;
+    size_t size = 0;
+    std::mutex mu;
+    std::condition_variable cv;
+    std::atomic<bool> stop{false}, awake{false};
+    std::atomic<long> turn{0};
+    std::atomic<int> left{0};
 };
 
 // A pass recorded instead of launched (the members of a group, see
@@ -71,6 +156,7 @@ struct st_ctx {
     std::vector<int> act_h;
     int nact = 0;                   // active slots, listed in s_list (launch grids cover these only)
     std::vector<hipGraphExec_t> graphs;   // one batch step, captured per active-slot count
+    Copiers *crew = nullptr;                    // threads of the large host transfers
     void *stage[2] = {nullptr, nullptr};        // pinned transfer buffers, made at the first large transfer
     hipEvent_t stage_ev[2] = {nullptr, nullptr};
     double *m_clk = nullptr;        // clock and dts of st_march (device), and its pinned host copy
@@ -500,6 +586,7 @@ extern "C" void st_ctx_destroy(st_ctx *c)
     if (c->td) (void)hipFree(c->td);
     if (c->red) (void)hipFree(c->red);
     if (c->red_h) (void)hipHostFree(c->red_h);
+    delete c->crew;
     for (int k = 0; k < 2; k++) {
         if (c->stage[k]) (void)hipHostFree(c->stage[k]);
         if (c->stage_ev[k]) (void)hipEventDestroy(c->stage_ev[k]);
@@ -590,8 +677,7 @@ bool last_stage(int scheme, int loop, int k)
 // Transfers of 1 MiB and more go through two pinned buffers of the context,
 // filled or emptied by several threads while the other is on the bus.  (The
 // runtime's own path for pageable memory copies, and takes the page faults of
-// a new array, on one thread: 19.7 MB up 558 -> 512 us, down 1068 -> 511, down
-// into a new array 1389 -> 884.)
+// a new array, on one thread: HOSTNUMBERS.)
 constexpr size_t STAGE_BYTES = 2 << 20, STAGE_MIN = 1 << 20;
 
 int stage_init(st_ctx *c)
@@ -600,20 +686,17 @@ int stage_init(st_ctx *c)
         if (!c->stage[k]) HIPCHK(c, hipHostMalloc(&c->stage[k], STAGE_BYTES));
         if (!c->stage_ev[k]) HIPCHK(c, hipEventCreateWithFlags(&c->stage_ev[k], hipEventDisableTiming));
     }
+    if (!c->crew) c->crew = new (std::nothrow) Copiers;
+    if (!c->crew) return fail(c, -3, "transfer threads: out of memory");
     return 0;
 }
 
-void par_copy(void *dst, const void *src, size_t n)
-{
-    constexpr long PIECE = 256 << 10;
-    const long pieces = (long)((n + PIECE - 1) / PIECE);
-    const int most = omp_get_max_threads() < 8 ? omp_get_max_threads() : 8;
-#pragma omp parallel for schedule(static) num_threads(pieces < most ? (int)pieces : most) if (pieces > 1)
-    for (long i = 0; i < pieces; i++) {
-        const size_t o = (size_t)i * PIECE, l = n - o < (size_t)PIECE ? n - o : (size_t)PIECE;
-        std::memcpy((char *)dst + o, (const char *)src + o, l);
-    }
-}
+// The threads awake for one transfer.
+struct Awake {
+    Copiers &crew;
+    explicit Awake(Copiers &c) : crew(c) { crew.begin(); }
+    ~Awake() { crew.end(); }
+};
 
 // The i-th piece of a transfer of nfields fields of w bytes, at most
 // STAGE_BYTES: several whole fields (rows > 1 device rows), or part of one.
@@ -649,11 +732,12 @@ int up(st_ctx *c, double *dev, const double *host, long nfields, int slot = 0)
     }
     TRY(stage_init(c));
     const long n = pieces_of(w, nfields);
+    const Awake on(*c->crew);
     for (long i = 0; i < n; i++) {
         const Piece p = piece(w, nfields, i);
         const int k = (int)(i & 1);
         HIPCHK(c, hipEventSynchronize(c->stage_ev[k]));       // the copy that last read this buffer
-        par_copy(c->stage[k], (const char *)host + p.field * w + p.off, p.bytes * p.rows);
+        c->crew->copy(c->stage[k], (const char *)host + p.field * w + p.off, p.bytes * p.rows);
         HIPCHK(c, hipMemcpy2DAsync(d + p.field * pitch + p.off, pitch, c->stage[k], p.bytes, p.bytes, p.rows,
                                    hipMemcpyHostToDevice, c->s));
         HIPCHK(c, hipEventRecord(c->stage_ev[k], c->s));
@@ -671,6 +755,7 @@ int down(st_ctx *c, double *host, const double *dev, long nfields, int slot = 0)
     } else {
         TRY(stage_init(c));
         const long n = pieces_of(w, nfields);
+        const Awake on(*c->crew);
         for (long i = 0; i <= n; i++) {
             if (i < n) {                                      // the next piece comes while the last is copied out
                 const Piece p = piece(w, nfields, i);
@@ -681,7 +766,7 @@ int down(st_ctx *c, double *host, const double *dev, long nfields, int slot = 0)
             if (i > 0) {
                 const Piece p = piece(w, nfields, i - 1);
                 HIPCHK(c, hipEventSynchronize(c->stage_ev[(i - 1) & 1]));
-                par_copy((char *)host + p.field * w + p.off, c->stage[(i - 1) & 1], p.bytes * p.rows);
+                c->crew->copy((char *)host + p.field * w + p.off, c->stage[(i - 1) & 1], p.bytes * p.rows);
             }
         }
     }

@@ -191,17 +191,16 @@ DEV Lane<M, P, NP, AL> make_lane(double *lds, int ss)
 }
 
 // Window of M own values plus H on each side, fetched from neighbours (W =
-// M + 2 H; H = 4 where the operator reaches that far, 2 for the periodic
-// derivatives).
-// On a non-periodic line the points beyond either end are the mirror
-// images f(-m) = f(m), f(n-1+m) = f(n-1-m) (the symmetry of
-// src/filters_nonperiodic1d.f:830-943); the compact operators overwrite
-// their closure rows and never read them.
+// M + 2 H; H = 4 where the operator reaches that far, 2 for the derivatives).
+// On a non-periodic line the points beyond either end of a full window are the
+// mirror images f(-m) = f(m), f(n-1+m) = f(n-1-m) (the symmetry of
+// src/filters_nonperiodic1d.f:830-943), for the Gaussian; the compact operators
+// overwrite their closure rows and never read them.
 template <int M, int W, int P, bool NP, bool AL>
 DEV void window(const double (&v)[M], const Lane<M, P, NP, AL> &L, double (&w)[W])
 {
     constexpr int H = (W - M) / 2;
-    static_assert(W == M + 2 * H && (!NP || H == HALO), "window width");
+    static_assert(W == M + 2 * H, "window width");
 #pragma unroll
     for (int k = 0; k < M; k++) w[H + k] = v[k];
 #pragma unroll
@@ -216,7 +215,7 @@ DEV void window(const double (&v)[M], const Lane<M, P, NP, AL> &L, double (&w)[W
         const int idx = o % M;
         w[H + M + o] = __shfl(v[idx], L.src(dl));
     }
-    if constexpr (NP) {
+    if constexpr (NP && H == HALO) {
         constexpr int n = M * P;
         // chunks whose window reaches past the first point: row -j sits
         // at w[HALO - c*M - j], its image row j at w[HALO - c*M + j]
@@ -243,10 +242,11 @@ DEV void window(const double (&v)[M], const Lane<M, P, NP, AL> &L, double (&w)[W
     }
 }
 
-// Half-width of the window that the derivatives need on a line: +-2, and
-// the full one on a non-periodic line (the closure rows reach further).
-template <bool NP>
-constexpr int d_halo() { return NP ? HALO : 2; }
+// Half-width of the window that the derivatives need on a line: +-2.  The
+// closure rows of a non-periodic line read the five points at its end, which
+// lie in the end chunk's window for 3 or more points per lane.
+template <bool NP, int M>
+constexpr int d_halo() { return NP && M < 3 ? HALO : 2; }
 
 // ---- cyclic solves ------------------------------------------------------
 //
@@ -603,6 +603,64 @@ DEV void np_fix(double (&x)[M], CTab &T, const Lane<M, P, NP, AL> &L)
     for (int k = 0; k < M; k++) x[k] -= z[k];
 }
 
+// The same for the derivatives on lines long enough that neither end is felt at
+// the other (rho^64 < 1e-26): the near rows' corrections then depend on the
+// first five values alone, the far rows' on the last five, and Z is geometric.
+// With L and U the recurrences of root rho truncated to the line (the scale
+// 1 + rho^2 folded in), column j = 0, 1 is scale rho^|k - j| / (1 - rho^2), and
+// from the far end, k counted from it, scale rho^k for the last row and scale
+// rho^(k - 1) (1 + rho^2) (k >= 1), scale rho (k = 0) for the one before.  Two
+// multiply-adds a point instead of a second solve with its scattered right-hand
+// side, some 250 vector instructions an operator.
+template <int OP, int M, int P, bool NP, bool AL>
+DEV void np_fix_ends(double (&x)[M], CTab &T, const Lane<M, P, NP, AL> &L)
+{
+    constexpr int n = M * P;
+    static_assert(OP < 2 && n >= 64, "derivatives on long lines");
+    const double rho = T.a1, scale = T.scale, r1 = 1.0 / rho;
+    double a[5], b[5];          // the five values at each end (M >= 5: in the end lanes only)
+#pragma unroll
+    for (int t = 0; t < 5; t++) {
+        if constexpr (M >= 5) {
+            a[t] = x[t];
+            b[t] = x[M - 5 + t];
+        } else {
+            a[t] = line_value<M, P>(x, L, t);
+            b[t] = line_value<M, P>(x, L, n - 5 + t);
+        }
+    }
+    double q[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const double *y = j < 2 ? a : b;
+        const int o = j < 2 ? 0 : 5;
+        double s = T.npG[j][o] * y[0];
+#pragma unroll
+        for (int t = 1; t < 5; t++) s = fma(T.npG[j][o + t], y[t], s);
+        q[j] = s;
+    }
+    const double g = scale / (1.0 - rho * rho);
+    double near = g * fma(q[1], r1, q[0]), far = scale * fma(q[2], r1 + rho, q[3]);
+    const double near0 = g * fma(q[1], rho, q[0]) - near, far0 = scale * fma(q[2], rho, q[3]) - far;   // at the end points
+    if constexpr (M >= 5) {
+        if constexpr (P == 64) {
+            near = rdlane<0>(near);
+            far = rdlane<63>(far);
+        } else {
+            near = __shfl(near, L.seg);
+            far = __shfl(far, L.seg + P - 1);
+        }
+    }
+    const double wn = near * T.lp[L.c][0], wf = far * T.lp[P - 1 - L.c][0];
+    x[0] -= L.c == 0 ? wn + near0 : wn;
+    x[M - 1] -= L.c == P - 1 ? wf + far0 : wf;
+#pragma unroll
+    for (int k = 1; k < M; k++) {
+        x[k] = fma(-T.cf[k - 1][0], wn, x[k]);
+        x[M - 1 - k] = fma(-T.cf[k - 1][0], wf, x[M - 1 - k]);
+    }
+}
+
 // Closure rows of the right-hand side.  OP 0: first derivative
 // (src/derivCDopt6_nonperiodic1d.f:463-471, 494-502, with the closure
 // constants of src/header:173-175), 1: second derivative (:615-629, 653-668),
@@ -652,10 +710,10 @@ DEV double closure_row(int r, const F &f)
 // Overwrite the closure rows (the first NB and last NB of the line) of the
 // right-hand side out = K * stencil.  The chunks that hold them are
 // enumerated at compile time so every window index is a constant.
-template <int OP, int M, int P, bool NP, bool AL>
-DEV void closure_rows(const double (&w)[M + 2 * HALO], double K, const Lane<M, P, NP, AL> &L, double (&out)[M])
+template <int OP, int M, int W, int P, bool NP, bool AL>
+DEV void closure_rows(const double (&w)[W], double K, const Lane<M, P, NP, AL> &L, double (&out)[M])
 {
-    constexpr int n = M * P, NB = OP == 2 ? 4 : 3;
+    constexpr int n = M * P, NB = OP == 2 ? 4 : 3, H = (W - M) / 2;
     // (selects, not branches: every index stays a constant)
 #pragma unroll
     for (int cc = 0; cc * M < NB; cc++) {
@@ -664,7 +722,7 @@ DEV void closure_rows(const double (&w)[M + 2 * HALO], double K, const Lane<M, P
         for (int k = 0; k < M; k++) {
             const int i = cc * M + k;
             if (i < NB) {
-                const int o = HALO - cc * M;
+                const int o = H - cc * M;
                 const double v = closure_row<OP>(i, [&](int j) { return w[o + j]; });
                 out[k] = here ? K * v : out[k];
             }
@@ -677,7 +735,7 @@ DEV void closure_rows(const double (&w)[M + 2 * HALO], double K, const Lane<M, P
         for (int k = 0; k < M; k++) {
             const int i = cc * M + k;
             if (i >= n - NB) {
-                const int o = HALO + n - 1 - cc * M;
+                const int o = H + n - 1 - cc * M;
                 const double v = closure_row<OP>(n - 1 - i, [&](int j) { return w[o - j]; });
                 out[k] = here ? K * (OP == 0 ? -v : v) : out[k];
             }
@@ -698,9 +756,10 @@ DEV void op_d1(const double (&w)[W], const Scale1 &K, CTab &T, const Lane<M, P, 
         const int i = k + H;
         out[k] = fma(K.a, w[i + 1] - w[i - 1], K.b * (w[i + 2] - w[i - 2]));
     }
-    if constexpr (NP) closure_rows<0>(w, K.k, L, out);
+    if constexpr (NP) closure_rows<0, M>(w, K.k, L, out);
     solve<0, M>(out, T, L);
-    if constexpr (NP) np_fix<0>(out, T, L);
+    if constexpr (NP && M * P >= 64) np_fix_ends<0>(out, T, L);
+    else if constexpr (NP) np_fix<0>(out, T, L);
 }
 
 // Second derivative: K.k = (N-1)^2*sx(2)*(1+rho^2), K.a, K.b, K.c its products
@@ -723,9 +782,10 @@ DEV void op_d2(const double (&w)[W], const Scale2 &K, CTab &T, const Lane<M, P, 
 #pragma unroll
         for (int k = 0; k < M; k++) out[k] = fma(K.c, x[k + HALO + 3] + x[k + HALO - 3], out[k]);
     }
-    if constexpr (NP) closure_rows<1>(w, K.k, L, out);
+    if constexpr (NP) closure_rows<1, M>(w, K.k, L, out);
     solve<1, M>(out, T, L);
-    if constexpr (NP) np_fix<1>(out, T, L);
+    if constexpr (NP && M * P >= 64) np_fix_ends<1>(out, T, L);
+    else if constexpr (NP) np_fix<1>(out, T, L);
 }
 
 // Eighth-order compact filter: K = 1/kappa.
@@ -739,7 +799,7 @@ DEV void op_filt(const double (&w)[M + 2 * HALO], const Coef &C, double K, CTab 
         out[k] = K * ((((C.f4 * (w[i + 4] + w[i - 4]) + C.f3 * (w[i + 3] + w[i - 3])) + C.f2 * (w[i + 2] + w[i - 2]))
                        + C.f1 * (w[i + 1] + w[i - 1])) + C.f0 * w[i]);
     }
-    if constexpr (NP) closure_rows<2>(w, K, L, out);
+    if constexpr (NP) closure_rows<2, M>(w, K, L, out);
     solve<2, M>(out, T, L);
     if constexpr (NP) np_fix<2>(out, T, L);
 }

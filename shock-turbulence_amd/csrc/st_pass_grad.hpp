@@ -139,7 +139,7 @@ struct PassGrad {
     template <int M, int P, bool NP, bool AL, class F, class A>
     DEV static void d1(const A &a, const Lane<M, P, NP, AL> &L, const F &f, double (&r)[M])
     {
-        double v[M], w[M + 2 * d_halo<NP>()];
+        double v[M], w[M + 2 * d_halo<NP, M>()];
 #pragma unroll
         for (int k = 0; k < M; k++) v[k] = f(k);
         window<M>(v, L, w);
@@ -218,7 +218,7 @@ struct PassGrad {
     DEV static void velocity(const A &a, const Lane<M, P, NP, AL> &L, const double (&mu)[M], double (&out)[5][M])
     {
         const double wd = i == DIR ? 4.0 / 3.0 + a.ph.bulk : 1.0;
-        constexpr int H = d_halo<NP>();
+        constexpr int H = d_halo<NP, M>();
         double v[M], w[M + 2 * H], r[M];
 #pragma unroll
         for (int k = 0; k < M; k++) v[k] = L.ld(i, k);
@@ -300,7 +300,7 @@ struct PassGrad {
         // D2(T)/gamma (the operator is linear).  CROSS: the store has mu' and
         // adds its term.
         {
-            constexpr int H = d_halo<NP>();
+            constexpr int H = d_halo<NP, M>();
             double v[M], w[M + 2 * H], r[M];
 #pragma unroll
             for (int k = 0; k < M; k++) v[k] = L.ld(3, k);
@@ -431,7 +431,7 @@ struct PassGrad {
     {
 #pragma unroll 1
         for (int m = 0; m < 2; m++) {
-            double f[M], w[M + 2 * d_halo<NP>()], r[M];
+            double f[M], w[M + 2 * d_halo<NP, M>()], r[M];
 #pragma unroll
             for (int k = 0; k < M; k++) f[k] = L.ld(m, k);
             window<M>(f, L, w);

@@ -15,7 +15,7 @@ struct PassLap2 : NoReuse {
     template <int M, int P, bool NP, bool AL, class A>
     DEV static void compute(const Geo &, const A &a, const Lane<M, P, NP, AL> &L, double (&out)[1][M])
     {
-        double f[M], w[M + 2 * d_halo<NP>()];
+        double f[M], w[M + 2 * d_halo<NP, M>()];
 #pragma unroll
         for (int k = 0; k < M; k++) f[k] = L.ld(0, k);
         window<M>(f, L, w);
@@ -29,7 +29,7 @@ struct PassLap2 : NoReuse {
 template <int M, int P, bool NP, bool AL, class A>
 DEV void d2_slot(const A &a, const Lane<M, P, NP, AL> &L, int m)
 {
-    double f[M], w[M + 2 * d_halo<NP>()], r[M];
+    double f[M], w[M + 2 * d_halo<NP, M>()], r[M];
 #pragma unroll
     for (int k = 0; k < M; k++) f[k] = L.ld(m, k);
     window<M>(f, L, w);

@@ -33,7 +33,7 @@ struct PassLapSE {
     {
 #pragma unroll 1
         for (int m = 0; m < 2; m++) {
-            double f[M], w[M + 2 * d_halo<NP>()], r[M];
+            double f[M], w[M + 2 * d_halo<NP, M>()], r[M];
 #pragma unroll
             for (int k = 0; k < M; k++) f[k] = L.ld(m, k);
             window<M>(f, L, w);

@@ -14,7 +14,7 @@ struct PassD1 : NoReuse {
     template <int M, int P, bool NP, bool AL, class A>
     DEV static void compute(const Geo &, const A &a, const Lane<M, P, NP, AL> &L, double (&out)[1][M])
     {
-        double f[M], w[M + 2 * d_halo<NP>()];
+        double f[M], w[M + 2 * d_halo<NP, M>()];
 #pragma unroll
         for (int k = 0; k < M; k++) f[k] = L.ld(0, k);
         window<M>(f, L, w);
@@ -34,7 +34,7 @@ struct PassD2 : NoReuse {
     template <int M, int P, bool NP, bool AL, class A>
     DEV static void compute(const Geo &, const A &a, const Lane<M, P, NP, AL> &L, double (&out)[1][M])
     {
-        double f[M], w[M + 2 * d_halo<NP>()], d2[M];
+        double f[M], w[M + 2 * d_halo<NP, M>()], d2[M];
 #pragma unroll
         for (int k = 0; k < M; k++) f[k] = L.ld(0, k);
         window<M>(f, L, w);

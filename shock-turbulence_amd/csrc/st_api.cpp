@@ -33,7 +33,7 @@ static_assert(st::K_NPASS <= KIND_RED, "pass kinds overlap the other timed kinds
 const char *kind_names[NKIND] = {
     "d1", "d2", "filter", "gauss", "grad", "lap_se",
     "lap2", "lap2_gauss", "gauss_eta", "gauss_hdiv", "hyper_div", "rk_filter", "filter_q",
-    "filter_q_fix", "grad_cross", "hdiv_rkf", "lap_se_lap2", "fq_grad", "", "", "", "reduce", "fill", ""};
+    "filter_q_fix", "grad_cross", "hdiv_rkf", "lap_se_lap2", "fq_grad", "vel_grad", "", "", "reduce", "fill", ""};
 
 struct Event {
     hipEvent_t a, b;
@@ -270,6 +270,7 @@ double kind_fields(int kind, int dir, const st::PassArgs &a)
     case st::K_D1: return a.iadd ? 3 : 2;
     case st::K_D2: return a.iadd ? 3 : 2;
     case st::K_FILT: return 2;
+    case st::K_VGRAD: return 4 + 3;
     case st::K_GAUSS: return 2;
     // Q, G of the direction, the dQ partial, the Lap e partial; z also reads
     // the two stored derivatives of its mixed terms
@@ -932,63 +933,66 @@ int op1(st_ctx *c, int kind, int dir, const double *in, double *out0, double *ou
     return pass(c, kind, dir, a, cadd);
 }
 
-// Compute_Laplacian (src/hyper_dynamic.f:41-58): out = D2z + D2x + D2y of f
-// (|.| with absval, :278-279); tmp holds 3 fields.
-int laplacian(st_ctx *c, const double *f, double *out, double *tmp, int absval)
-{
-    const long N = c->N;
-    TRY(op1(c, st::K_D2, 0, f, nullptr, tmp, 0, 1.0));
-    TRY(op1(c, st::K_D2, 1, f, nullptr, tmp + N, 0, 1.0));
-    TRY(op1(c, st::K_D2, 2, f, nullptr, tmp + 2 * N, 0, 1.0));
-    return kerr(c, st::run_sum3(tmp + 2 * N, tmp, tmp + N, c->ni, absval, out, c->s), "laplacian sum");
-}
-
 // Compute_hyper (src/hyper_dynamic.f:173-318; with a non-periodic x the
 // static coefficients of src/hyper_routines.f:66-214) for one slot, outside
 // a stage: beta*, mu*, kappa* into Hc from the resident state and, with
 // use_grad, the velocity gradients in G (/GRAD/ as the last RHS left it);
 // without, |S| = 0, as at a start before any RHS (src/main.f:100 with
-// /GRAD/ still zero).  Scratch: the 10 partial-sum fields and T5, which a
-// stage rewrites before reading.
+// /GRAD/ still zero).  The passes are those of a stage, on fields of their own:
+// the 19 of T5, tB, tC, dQp and L2ep, which follow each other and which a stage
+// rewrites before reading (what st_rhs leaves for st_hyper_rhs stays as it is).
+// 17 launches (35 as single operators and sums).
 int seq_compute_hyper(st_ctx *c, int slot, int use_grad)
 {
     const long off = (long)slot * c->ni, N = c->N, ni = c->ni;
-    const double *Q = c->Q + off;
-    double *W = c->dQp + off;
-    double *T = c->T5 + off;
-    TRY(kerr(c, st::run_hyp_prep(Q, use_grad ? c->G + off : nullptr, N, ni, 1, W, c->s), "hyper prep"));
+    double *X = c->T5 + off, *e = X + N, *vg = X + 6 * N;
+    st::PassArgs a = base_args(c);
+    a.Q = c->Q + off;
+    a.S = X;
+    a.L2e = X + 2 * N;
+    a.L2S = X + 3 * N;
+    a.L4e = X + 4 * N;
+    a.L4S = X + 5 * N;
+    a.eta = c->eta + off;
+    TRY(kerr(c, st::run_hyp_prep(a.Q, use_grad ? c->G + off : nullptr, N, ni, a.S, e, c->s), "hyper prep"));
     double *Cb = nullptr;
     if (!c->g.nonperiodic_x) {
-        // Compute_coeff1 (:72-165): vorticity W[3..5] and dilatation W[6] of U
-        double *U0 = W, *U1 = W + N, *U2 = W + 2 * N;
-        double *wx = W + 3 * N, *wy = W + 4 * N, *wz = W + 5 * N, *dil = W + 6 * N;
-        TRY(op1(c, st::K_D1, 1, U2, wx, nullptr, 0, 1.0));            // :105-106
-        TRY(op1(c, st::K_D1, 2, U1, wx, nullptr, 1, -1.0));
-        TRY(op1(c, st::K_D1, 0, U2, wy, nullptr, 0, -1.0));           // :114-115
-        TRY(op1(c, st::K_D1, 2, U0, wy, nullptr, 1, 1.0));
-        TRY(op1(c, st::K_D1, 0, U1, wz, nullptr, 0, 1.0));            // :123-124
-        TRY(op1(c, st::K_D1, 1, U0, wz, nullptr, 1, -1.0));
-        TRY(op1(c, st::K_D1, 0, U0, dil, nullptr, 0, 1.0));           // :132-140
-        TRY(op1(c, st::K_D1, 1, U1, dil, nullptr, 1, 1.0));
-        TRY(op1(c, st::K_D1, 2, U2, dil, nullptr, 1, 1.0));
+        // Compute_coeff1 (:72-165) from the gradients of this state
+        for (int d = 0; d < 3; d++) {
+            st::PassArgs g = a;
+            g.out0 = vg + 3 * d * N;
+            TRY(pass(c, st::K_VGRAD, d, g));
+        }
         Cb = c->Cb + off;
-        TRY(kerr(c, st::run_hyp_cb(W, N, ni, Cb, c->s), "C_beta"));
+        TRY(kerr(c, st::run_hyp_cb(vg, N, ni, Cb, c->s), "C_beta"));
     }
-    // |Lap^2 S| into W[7], |Lap^2 e| into W[8] (:272-279)
-    TRY(laplacian(c, W + 7 * N, W + 9 * N, T, 0));
-    TRY(laplacian(c, W + 9 * N, W + 7 * N, T, 1));
-    TRY(laplacian(c, W + 8 * N, W + 9 * N, T, 0));
-    TRY(laplacian(c, W + 9 * N, W + 8 * N, T, 1));
-    // eta (:284-297), Gaussian x, y, z (:300), the coefficients (:303-314)
-    double *eta = c->eta + off;
-    TRY(kerr(c, st::run_hyp_eta(Q, N, ni, c->ph, W + 7 * N, W + 8 * N, eta, c->s), "eta"));
-    TRY(op1(c, st::K_GAUSS, 0, eta, T, nullptr, 0, 1.0));
-    TRY(op1(c, st::K_GAUSS, 1, T, T + N, nullptr, 0, 1.0));
-    TRY(op1(c, st::K_GAUSS, 2, T + N, W + 9 * N, nullptr, 0, 1.0));
-    TRY(op1(c, st::K_GAUSS, 0, eta + N, T + 2 * N, nullptr, 0, 1.0));
-    TRY(op1(c, st::K_GAUSS, 1, T + 2 * N, T + 3 * N, nullptr, 0, 1.0));
-    TRY(op1(c, st::K_GAUSS, 2, T + 3 * N, W + 7 * N, nullptr, 0, 1.0));
-    return kerr(c, st::run_hyp_coef(W + 9 * N, W + 7 * N, Cb, N, ni, c->ph, c->Hc + off, c->s), "coefficients");
+    // Lap e, then Lap|S| and Lap(Lap e) as a stage forms them (:272-279)
+    {
+        st::PassArgs l = a;
+        l.L2S = e;
+        l.L4S = a.L2e;
+        for (int d = 0; d < 3; d++) {
+            l.first = d == 0;
+            TRY(pass(c, st::K_LAP2, d, l));
+        }
+        l.first = 1;
+        l.L2S = a.S;
+        l.L4S = a.L2S;
+        TRY(pass(c, st::K_LAP2, 1, l));
+        l.L2S = a.L2e;
+        l.L4S = a.L4e;
+        TRY(pass(c, st::K_LAP2, 1, l));
+    }
+    TRY(pass(c, st::K_LAPSE, 0, a));
+    TRY(pass(c, st::K_LAPSE_LAP2, 2, a));
+    // |Lap^2 S|, |Lap^2 e|, eta (:284-297), Gaussian y, x, z (:300), the
+    // coefficients (:303-314)
+    TRY(pass(c, st::K_LAP2, 0, a));
+    TRY(pass(c, st::K_LAP2_LAST, 1, a));
+    TRY(pass(c, st::K_GAUSS_ETA, 0, a));
+    TRY(op1(c, st::K_GAUSS, 2, a.eta, X, nullptr, 0, 1.0));
+    TRY(op1(c, st::K_GAUSS, 2, a.eta + N, X + N, nullptr, 0, 1.0));
+    return kerr(c, st::run_hyp_coef(X, X + N, Cb, N, ni, c->ph, c->Hc + off, c->s), "coefficients");
 }
 
 int stage_loop(st_ctx *c, double dt, double *time, int *step)
@@ -1180,11 +1184,12 @@ extern "C" int st_compute_grad(st_ctx *c, double *maxdil, double *enstrophy)
 {
     if (!c) return -1;
     const long N = c->N, ni = c->ni;
-    double *W = c->dQp;
-    TRY(kerr(c, st::run_hyp_prep(c->Q, nullptr, N, ni, 0, W, c->s), "grad prep"));
     // /GRAD/ velocity gradients G[(3d + i) N] = d u_i / d x_d (src/grad.f:55-96)
-    for (int d = 0; d < 3; d++)
-        for (int i = 0; i < 3; i++) TRY(op1(c, st::K_D1, d, W + i * N, c->G + (3 * d + i) * N, nullptr, 0, 1.0));
+    for (int d = 0; d < 3; d++) {
+        st::PassArgs a = base_args(c);
+        a.out0 = c->G + 3 * d * N;
+        TRY(pass(c, st::K_VGRAD, d, a));
+    }
     TRY(kerr(c, st::run_gradred(c->G, N, ni, c->red, c->s), "grad reductions"));
     const int nb = st::gradred_blocks(ni);
     HIPCHK(c, hipMemcpyAsync(c->red_h, c->red, sizeof(double) * 2 * nb, hipMemcpyDeviceToHost, c->s));

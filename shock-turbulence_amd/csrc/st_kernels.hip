@@ -56,7 +56,7 @@ void pass_default_cfg(int kind, int dir, const DirTab &wide, long ni, long N, in
 hipError_t run_pass(int kind, const DirTab &t, int nt, int dir, int My, int Mz, int Mx, const PassArgs &a, hipStream_t s)
 {
     switch (kind) {
-    case K_D1: case K_D2: case K_FILT: case K_GAUSS:
+    case K_D1: case K_D2: case K_FILT: case K_GAUSS: case K_VGRAD:
         return launch_ops(kind, t, nt, dir, My, Mz, Mx, a, s);
     // x first (no mixed terms), z with two, y last with four and the
     // pointwise assembly
@@ -372,20 +372,14 @@ hipError_t run_sponge(const PassArgs &a, const double *spg, int Mx, int nleft, h
 // slot: the pointers already carry the slot's offset, fields are N apart.
 // ---------------------------------------------------------------------
 
-// W[0..2] = Q_i * (1/rho) (src/hyper_dynamic.f:87-97, src/grad.f:40-48);
-// with want_hyp also W[7] = |S| of the symmetrised /GRAD/ (0 when G is
-// null: the coefficients of a start without gradients, src/main.f:100)
-// (src/hyper_dynamic.f:227-245, :12-33) and W[8] = e (:251-266).
-__global__ void __launch_bounds__(256) k_hyp_prep(const double *Q, const double *G, long N, long ni, int want_hyp,
-                                                  double *W)
+// |S| of the symmetrised /GRAD/ (0 when G is null: the coefficients of a
+// start without gradients, src/main.f:100) (src/hyper_dynamic.f:227-245,
+// :12-33) and e (:251-266).
+__global__ void __launch_bounds__(256) k_hyp_prep(const double *Q, const double *G, long N, long ni, double *S, double *e)
 {
     for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < ni; i += (long)gridDim.x * blockDim.x) {
         const double q1 = Q[i], q2 = Q[N + i], q3 = Q[2 * N + i], q4 = Q[3 * N + i];
         const double t = 1.0 / q4;
-        W[i] = q1 * t;
-        W[N + i] = q2 * t;
-        W[2 * N + i] = q3 * t;
-        if (!want_hyp) continue;
         double s = 0.0;
         if (G) {
             const double s11 = G[i], s22 = G[4 * N + i], s33 = G[8 * N + i];
@@ -394,44 +388,21 @@ __global__ void __launch_bounds__(256) k_hyp_prep(const double *Q, const double 
             const double s23 = 0.5 * (G[7 * N + i] + G[5 * N + i]);
             s = sqrt(0.5 * (s11 * s11 + s22 * s22 + s33 * s33 + 2.0 * (s12 * s12 + s13 * s13 + s23 * s23)));
         }
-        W[7 * N + i] = s;
-        W[8 * N + i] = t * (Q[4 * N + i] - 0.5 * t * (q1 * q1 + q2 * q2 + q3 * q3));
+        S[i] = s;
+        e[i] = t * (Q[4 * N + i] - 0.5 * t * (q1 * q1 + q2 * q2 + q3 * q3));
     }
 }
 
-// C_beta from the vorticity W[3..5] and dilatation W[6]
-// (src/hyper_dynamic.f:142-160)
-__global__ void __launch_bounds__(256) k_hyp_cb(const double *W, long N, long ni, double *Cb)
+// C_beta from the nine velocity gradients g[3d + i] = du_i/dx_d: vorticity and
+// dilatation (src/hyper_dynamic.f:105-160)
+__global__ void __launch_bounds__(256) k_hyp_cb(const double *g, long N, long ni, double *Cb)
 {
     for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < ni; i += (long)gridDim.x * blockDim.x) {
-        const double g1 = W[3 * N + i], g2 = W[4 * N + i], g3 = W[5 * N + i], g4 = W[6 * N + i];
+        const double g1 = g[5 * N + i] - g[7 * N + i], g2 = g[6 * N + i] - g[2 * N + i], g3 = g[N + i] - g[3 * N + i];
+        const double g4 = (g[i] + g[4 * N + i]) + g[8 * N + i];
         const double fac = 0.5 * (1.0 - tanh(2.5 + 10.0 * g4));
         const double om2 = g1 * g1 + g2 * g2 + g3 * g3;
         Cb[i] = fac * g4 * g4 / (g4 * g4 + om2 + 1.0e-7) + 1.0e-20;
-    }
-}
-
-// Compute_Laplacian's sum d2S = D2z + D2x + D2y (src/hyper_dynamic.f:54),
-// optionally |.| (:278-279)
-__global__ void __launch_bounds__(256) k_sum3(const double *z, const double *x, const double *y, long ni, int absval,
-                                              double *out)
-{
-    for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < ni; i += (long)gridDim.x * blockDim.x) {
-        const double s = z[i] + x[i] + y[i];
-        out[i] = absval ? fabs(s) : s;
-    }
-}
-
-// eta_1 = rho |Lap^2 S|, eta_2 = (rho/T) c |Lap^2 e| (src/hyper_dynamic.f:284-297)
-__global__ void __launch_bounds__(256) k_hyp_eta(const double *Q, long N, long ni, Phys ph, const double *d4S,
-                                                 const double *d4e, double *eta)
-{
-    for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < ni; i += (long)gridDim.x * blockDim.x) {
-        const double q4 = Q[3 * N + i];
-        const Prim pr = prim(ph, Q[i], Q[N + i], Q[2 * N + i], q4, Q[4 * N + i]);
-        const double fac3 = (q4 / pr.T) * sqrt(ph.gamma * pr.p * pr.vs);
-        eta[i] = q4 * d4S[i];
-        eta[N + i] = fac3 * d4e[i];
     }
 }
 
@@ -490,28 +461,15 @@ static long pw_blocks(long ni)
     return b > 4096 ? 4096 : b;
 }
 
-hipError_t run_hyp_prep(const double *Q, const double *G, long N, long ni, int want_hyp, double *W, hipStream_t s)
+hipError_t run_hyp_prep(const double *Q, const double *G, long N, long ni, double *S, double *e, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_hyp_prep, dim3((unsigned)pw_blocks(ni)), dim3(256), 0, s, Q, G, N, ni, want_hyp, W);
+    hipLaunchKernelGGL(k_hyp_prep, dim3((unsigned)pw_blocks(ni)), dim3(256), 0, s, Q, G, N, ni, S, e);
     return hipGetLastError();
 }
 
-hipError_t run_hyp_cb(const double *W, long N, long ni, double *Cb, hipStream_t s)
+hipError_t run_hyp_cb(const double *g, long N, long ni, double *Cb, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_hyp_cb, dim3((unsigned)pw_blocks(ni)), dim3(256), 0, s, W, N, ni, Cb);
-    return hipGetLastError();
-}
-
-hipError_t run_sum3(const double *z, const double *x, const double *y, long ni, int absval, double *out, hipStream_t s)
-{
-    hipLaunchKernelGGL(k_sum3, dim3((unsigned)pw_blocks(ni)), dim3(256), 0, s, z, x, y, ni, absval, out);
-    return hipGetLastError();
-}
-
-hipError_t run_hyp_eta(const double *Q, long N, long ni, const Phys &ph, const double *d4S, const double *d4e,
-                       double *eta, hipStream_t s)
-{
-    hipLaunchKernelGGL(k_hyp_eta, dim3((unsigned)pw_blocks(ni)), dim3(256), 0, s, Q, N, ni, ph, d4S, d4e, eta);
+    hipLaunchKernelGGL(k_hyp_cb, dim3((unsigned)pw_blocks(ni)), dim3(256), 0, s, g, N, ni, Cb);
     return hipGetLastError();
 }
 

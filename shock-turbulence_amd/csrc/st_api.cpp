@@ -492,16 +492,12 @@ extern "C" int st_batch_create(const st_grid *grid, const st_params *params, int
             }
         }
     }
-    // non-periodic lines: the boundary correction's registers make wide tiles
-    // lose in the passes with several solves per point (512 x 192 x 192: x
-    // gradient 7417 us a stage on 256 threads, 7626 on 512); the others take
-    // their shape up to 512 threads (7404 -> 7300 together)
+    // non-periodic lines: the boundary correction's registers leave 1024
+    // threads too few; 512 it is (512 x 192 x 192, x gradient: 7061 us a stage
+    // on 256 threads, 6767 on 512)
     if (grid->nonperiodic_x && !getenv("ST_NT1024"))
-        for (int k = 0; k < NKIND; k++) {
-            const bool light = k == st::K_LAPSE || k == st::K_LAP2 || k == st::K_GAUSS_ETA || k == st::K_HDIV;
-            const int most = light ? 512 : 256;
-            if (c->cfg_nt[k][0] > most) c->cfg_nt[k][0] = most;
-        }
+        for (int k = 0; k < NKIND; k++)
+            if (c->cfg_nt[k][0] > 512) c->cfg_nt[k][0] = 512;
     hipError_t e;
     if ((e = hipStreamCreateWithFlags(&c->s, hipStreamNonBlocking)) != hipSuccess) {
         fail(c, -3, "hipStreamCreate: %s", hipGetErrorString(e));

@@ -205,9 +205,9 @@ struct PassGaussEta : NoReuse {
 // are written for their passes, which then read four fields each instead of
 // the coefficients, eight gradients and the state.  The pass is bound by
 // memory: 34 fields a point (37 with the coefficients written, which only
-// the last stage of a step needs).  256^3: this pass 0.74 -> 0.86 ms at 26 ->
-// 34 fields, the x pass 0.69 -> 0.34 ms (23 -> 12), the y pass 0.96 -> 0.80
-// ms (36 -> 29).
+// the last stage of a step needs).  256^3: this pass 745 -> 895 us at 26 ->
+// 34 fields, the x pass 698 -> 336 us (23 -> 12), the y pass 959 -> 703 us
+// (36 -> 29, streamed).
 //   compute   Gaussian along z of the two eta fields
 //   mid       per point: beta*, mu*, kappa*, the x and y fluxes (written),
 //             the staged z fluxes

@@ -32,11 +32,15 @@ HBM_PEAK_GBS = 8000.0   # MI355X HBM3E
 STAGES_PER_STEP = 11
 
 # kernel template of each pass kind (csrc/st_pass_*.hip)
+# pass kind -> (struct, stream bits of its launches on large grids)
 PASS_STRUCT = {
-    "lap2": "PassLap2", "lap2_gauss": "PassLap2Gauss", "lap_se_lap2": "PassLapSELap2", "gauss_eta": "PassGaussEta",
-    "gauss_hdiv": "PassGaussHdiv", "hyper_div": "PassHyperDiv", "rk_filter": "PassFilterQ<0>",
-    "filter_q": "PassFilterQ<1>", "filter_q_fix": "PassFilterQ<2>", "hdiv_rkf": "PassHdivRkf",
+    "fq_grad": ("PassFqGrad", 3), "lap_se": ("PassLapSE", 1), "lap2": ("PassLap2", 1),
+    "lap2_gauss": ("PassLap2Gauss", 7), "lap_se_lap2": ("PassLapSELap2", 1), "gauss_eta": ("PassGaussEta", 1),
+    "gauss_hdiv": ("PassGaussHdiv", 3), "hyper_div": ("PassHyperDiv", 1), "rk_filter": ("PassFilterQ<0>", 0),
+    "filter_q": ("PassFilterQ<1>", 0), "filter_q_fix": ("PassFilterQ<2>", 0), "hdiv_rkf": ("PassHdivRkf", 7),
+    "grad_cross": ("PassGrad<1, 2, false>", 7),
 }
+STREAM_POINTS, STREAM_Y = 3 << 19, 4
 
 
 def kernel_symbol(kind, d, narrow, nt, n):
@@ -47,18 +51,18 @@ def kernel_symbol(kind, d, narrow, nt, n):
     if narrow and 2 * P <= 64:
         M, P = M // 2, 2 * P
     if kind == "grad" and d == "x":
-        st = "PassGrad<0, 1, false>"
+        st, bits = "PassGrad<0, 1, false>", 3
     elif kind == "grad":
-        st = "PassGrad<2, 2, true>" if nt == 256 and M == 8 and P == 32 else "PassGrad<2, 1, false>"
-    elif kind == "grad_cross":
-        st = "PassGrad<1, 2, false>"
-    elif kind == "lap_se":
-        st = "PassLapSE<%s>" % ("false" if d == "x" else "true")
+        two = P == 32 and (M == 8 if nt == 256 else nt == 512 and 4 <= M <= 7)
+        st, bits = ("PassGrad<2, 2, true>", 3) if two else ("PassGrad<2, 1, false>", 0)
+    elif kind in PASS_STRUCT:
+        st, bits = PASS_STRUCT[kind]
     else:
-        st = PASS_STRUCT.get(kind)
-        if st is None:
-            return kind
-    return "k_pass<%d, %d, %d, false, %s>" % (M, P, nt, st)
+        return kind
+    # large grids stream: passes that name y, the others on 16 lines a tile and more
+    if n ** 3 < STREAM_POINTS or not (bits & STREAM_Y or nt // P >= 16):
+        bits = 0
+    return "k_pass<%d, %d, %d, false, %s, %d>" % (M, P, nt, st, bits)
 
 
 def traffic_of(kernel):

@@ -920,18 +920,6 @@ int kerr(st_ctx *c, hipError_t e, const char *what)
     return 0;
 }
 
-// One single-operator pass over one slot's fields (the pointers carry the
-// slot's offset; the launch covers slot 0 of a one-slot argument set).
-int op1(st_ctx *c, int kind, int dir, const double *in, double *out0, double *out1, int iadd, double cadd)
-{
-    st::PassArgs a = base_args(c);
-    a.in0 = in;
-    a.out0 = out0;
-    a.out1 = out1;
-    a.iadd = iadd;
-    return pass(c, kind, dir, a, cadd);
-}
-
 // Compute_hyper (src/hyper_dynamic.f:173-318; with a non-periodic x the
 // static coefficients of src/hyper_routines.f:66-214) for one slot, outside
 // a stage: beta*, mu*, kappa* into Hc from the resident state and, with
@@ -989,8 +977,12 @@ int seq_compute_hyper(st_ctx *c, int slot, int use_grad)
     TRY(pass(c, st::K_LAP2, 0, a));
     TRY(pass(c, st::K_LAP2_LAST, 1, a));
     TRY(pass(c, st::K_GAUSS_ETA, 0, a));
-    TRY(op1(c, st::K_GAUSS, 2, a.eta, X, nullptr, 0, 1.0));
-    TRY(op1(c, st::K_GAUSS, 2, a.eta + N, X + N, nullptr, 0, 1.0));
+    for (int j = 0; j < 2; j++) {
+        st::PassArgs z = a;
+        z.in0 = a.eta + j * N;
+        z.out0 = X + j * N;
+        TRY(pass(c, st::K_GAUSS, 2, z));
+    }
     return kerr(c, st::run_hyp_coef(X, X + N, Cb, N, ni, c->ph, c->Hc + off, c->s), "coefficients");
 }
 

@@ -137,7 +137,10 @@ int st_rk_stage(st_ctx *ctx, double alpha, double beta, double dt, int reset_qw)
 /* LDDRK4(time, step)  src/lddrk4_periodic_sf.f:311 with a given dt. */
 int st_step(st_ctx *ctx, double dt, double *time, int *step);
 /* nsteps of march mode 1 (src/main.f:129-136): Compute_CFL, Compute_Tstep,
- * LDDRK4 per step.  dt_out (may be NULL) receives each step's dt. */
+ * LDDRK4 per step.  dt_out (may be NULL) receives each step's dt.  A dt that
+ * is not positive and finite ends the march before its step (-5): state,
+ * /HYPER/ and /GRAD/ are as that dt found them, *time and *step those of the
+ * steps before. */
 int st_march(st_ctx *ctx, int nsteps, double *time, int *step, double *dt_out);
 /* Compute_Mom, Compute_KE, Compute_Mass, Compute_Energy, Compute_Entropy
  * (src/lddrk4_periodic_sf.f:153-302): MomX MomY MomZ KE Mass Energy Entropy. */

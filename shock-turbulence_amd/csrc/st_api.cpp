@@ -8,6 +8,7 @@
 #include <cstdlib>
 #include <array>
 #include <atomic>
+#include <chrono>
 #include <condition_variable>
 #include <cstring>
 #include <exception>
@@ -26,6 +27,7 @@ namespace {
 constexpr int NKIND = 24;          // pass kinds + reductions + fills
 constexpr int KIND_RED = 21, KIND_FILL = 22;
 constexpr int MARCH_CHUNK = 256;   // steps of st_march between host synchronisations
+constexpr int MARCH_AHEAD = 2;     // steps of st_march that the host enqueues before the device's
 static_assert(st::K_NPASS <= KIND_RED, "pass kinds overlap the other timed kinds");
 
 // Fields read + written per point by one launch of each kind (RMW counts
@@ -120,6 +122,18 @@ private:
     std::atomic<int> left{0};
 };
 
+// The clock block of st_march: time, dt, the last dt, four integers, then the
+// dt of each step of a chunk.
+struct MarchClock {
+    double *time, *dt, *dt_last;
+    int *act, *run, *target, *step;
+    double *hist;
+    explicit MarchClock(double *p)
+        : time(p), dt(p + 1), dt_last(p + 2), act((int *)(p + 3)), run(act + 1), target(act + 2), step(act + 3), hist(p + 5)
+    {
+    }
+};
+
 // A pass recorded instead of launched (the members of a group, see
 // group_step): its kind, direction, prepared arguments and host tables.
 struct Rec {
@@ -159,8 +173,9 @@ struct st_ctx {
     Copiers *crew = nullptr;                    // threads of the large host transfers
     void *stage[2] = {nullptr, nullptr};        // pinned transfer buffers, made at the first large transfer
     hipEvent_t stage_ev[2] = {nullptr, nullptr};
-    double *m_clk = nullptr;        // clock and dts of st_march (device), and its pinned host copy
+    double *m_clk = nullptr;        // clock and dts of st_march (MarchClock, device), and its pinned host copy
     double *m_clk_h = nullptr;
+    int *m_seen = nullptr;          // pinned, written by the device: steps of the chunk with a dt, -1 once one was refused
     double *spg = nullptr;          // sponge: sigma per x index, then the left and right reference states
     int spg_left = 0;               // x indices [0, spg_left) take the left reference state
     int use_graph = 1;
@@ -516,6 +531,7 @@ extern "C" int st_batch_create(const st_grid *grid, const st_params *params, int
         (e = hipHostMalloc(&c->red_h, sizeof(double) * c->red_n)) != hipSuccess ||
         (e = hipMalloc(&c->m_clk, sizeof(double) * (5 + MARCH_CHUNK))) != hipSuccess ||
         (e = hipHostMalloc(&c->m_clk_h, sizeof(double) * (5 + MARCH_CHUNK))) != hipSuccess ||
+        (e = hipHostMalloc(&c->m_seen, sizeof(int), hipHostMallocCoherent)) != hipSuccess ||
         (e = hipMalloc(&sp, ns * (6 * sizeof(int) + 4 * sizeof(double)))) != hipSuccess) {
         fail(c, -3, "device allocation: %s", hipGetErrorString(e));
         *out = c;
@@ -590,6 +606,7 @@ extern "C" void st_ctx_destroy(st_ctx *c)
     }
     if (c->m_clk) (void)hipFree(c->m_clk);
     if (c->m_clk_h) (void)hipHostFree(c->m_clk_h);
+    if (c->m_seen) (void)hipHostFree(c->m_seen);
     if (c->s) (void)hipStreamDestroy(c->s);
     delete c;
 }
@@ -849,15 +866,12 @@ int seq_hyper(st_ctx *c, const st::PassArgs &base, const st::PassArgs *rk = null
 // is not its first (have_x) or not its last (!last) shares the x pass between
 // them with its neighbour.  last: the coefficients /HYPER/ are left in Hc (the
 // stages before the last of a step rewrite them before anything reads them).
-// guard: a run flag for the passes that write the state alone (the others
-// then start without waiting for a flag).
 int seq_stage(st_ctx *c, const st::PassArgs &base0, double ra, double rb, double dt, bool have_x = false,
-              bool last = true, const int *guard = nullptr)
+              bool last = true)
 {
     st::PassArgs base = base0;
     base.keep_hc = last ? 1 : 0;
     st::PassArgs a = base;
-    if (guard) a.act = guard;
     a.rk_a = ra;
     a.rk_b = rb;
     a.dt = dt;
@@ -1018,7 +1032,7 @@ int batch_step(st_ctx *c)
     hipError_t err = st::run_cfl_tstep(a, pc, c->p.hyper_param == 1 ? pt : nullptr, &nb, c->s);
     if (err == hipSuccess)
         err = st::run_dt(pc, pt, nb, c->ns, c->s_act, c->s_target, c->s_step, c->p.cfl_cal, c->p.hyper_param,
-                         c->g.nonperiodic_x ? 1 : 0, c->s_run, c->s_dt, c->s_dtlast, nullptr, 0, c->s);
+                         c->g.nonperiodic_x ? 1 : 0, c->s_run, c->s_dt, c->s_dtlast, nullptr, 0, nullptr, c->s);
     if (err != hipSuccess) return fail(c, -4, "batch dt: %s", hipGetErrorString(err));
     a.act = c->s_run;
     a.sre = c->s_re;
@@ -1273,55 +1287,87 @@ extern "C" int st_step(st_ctx *c, double dt, double *time, int *step)
     return 0;
 }
 
+namespace {
+
+// Enqueue one step of st_march: its dt, then the stages of both loops.
+int march_step(st_ctx *c, const st::PassArgs &a, const MarchClock &m, int step0)
+{
+    const int hyper = c->p.hyper_param;
+    double *pc = c->red, *pt = c->red + (long)st::reduce_blocks(c->ni) * c->ns * 2;
+    int nb = 0;
+    Event e;
+    if (c->prof) prof_begin(c, KIND_RED * 3, e);
+    hipError_t err = st::run_cfl_tstep(base_args(c), pc, hyper == 1 ? pt : nullptr, &nb, c->s);
+    if (err == hipSuccess)
+        err = st::run_dt(pc, pt, nb, 1, m.act, m.target, m.step, c->p.cfl_cal, hyper, c->g.nonperiodic_x ? 1 : 0, m.run,
+                         m.dt, m.dt_last, m.hist, step0, c->m_seen, c->s);
+    if (c->prof) prof_end(c, e);
+    if (err != hipSuccess) return fail(c, -4, "march dt: %s", hipGetErrorString(err));
+    for (int loop = 0; loop < 2; loop++) {
+        const double *ra, *rb;
+        const int ns = rk_loop(c->p.rk_scheme, loop, &ra, &rb);
+        if (!ns) break;
+        for (int k = 0; k < ns; k++)                         // (QW: as stage_loop)
+            TRY(seq_stage(c, a, ra[k], rb[k], 0.0, loop || k, last_stage(c->p.rk_scheme, loop, k)));
+        err = st::run_clock(1, m.run, m.dt, m.time, m.step, last_stage(c->p.rk_scheme, loop, ns - 1), c->s);
+        if (err != hipSuccess) return fail(c, -4, "march clock: %s", hipGetErrorString(err));
+    }
+    return 0;
+}
+
+// Wait until the device has decided on `steps` steps of a chunk; false once
+// it has refused one (or the stream has stopped on an error).
+bool march_seen(st_ctx *c, int steps)
+{
+    for (;;) {
+        const int v = __atomic_load_n(c->m_seen, __ATOMIC_ACQUIRE);
+        if (v < 0) return false;
+        if (v >= steps) return true;
+        const hipError_t e = hipStreamQuery(c->s);
+        if (e != hipErrorNotReady) return e == hipSuccess && __atomic_load_n(c->m_seen, __ATOMIC_ACQUIRE) >= steps;
+        std::this_thread::sleep_for(std::chrono::microseconds(20));
+    }
+}
+
+}  // namespace
+
 // March of one run with its dt formed on the device, as a batch's: no host
 // round trip between the steps (each cost two synchronising copies).  The
 // run's clock lives in its own device block (a batch's slot 0 keeps its own);
-// the dts come back once per MARCH_CHUNK steps.
+// the dts come back once per MARCH_CHUNK steps.  A dt that is not positive and
+// finite ends the run: the passes then leave all they write as it is (their
+// run flag, which every pass waits for: 32^3 1814 us a two-step march without,
+// 1837 with; 256^3 the same), and the host, which stays MARCH_AHEAD steps
+// before the device, enqueues no more.
 extern "C" int st_march(st_ctx *c, int nsteps, double *time, int *step, double *dt_out)
 {
     if (!c || !time || !step) return -1;
+    const MarchClock m(c->m_clk);
     st::PassArgs a = base_args(c);
-    double *tm = c->m_clk, *dt = c->m_clk + 1, *dt_last = c->m_clk + 2;
-    int *ints = (int *)(c->m_clk + 3);
-    int *act = ints, *run = ints + 1, *target = ints + 2, *stepc = ints + 3;
-    double *hist = c->m_clk + 5;
-    a.sdt = dt;
-    const int hyper = c->p.hyper_param, first = c->g.nonperiodic_x ? 1 : 0;
-    double *pc = c->red, *pt = c->red + (long)st::reduce_blocks(c->ni) * c->ns * 2;
+    a.sdt = m.dt;
+    a.act = m.run;
     for (int done = 0; done < nsteps;) {
         const int n = nsteps - done < MARCH_CHUNK ? nsteps - done : MARCH_CHUNK;
         const int step0 = *step;
-        hipError_t err = st::run_clock_set(act, target, stepc, tm, n, step0, *time, c->s);
+        __atomic_store_n(c->m_seen, 0, __ATOMIC_RELEASE);     // (the stream's earlier marches have been waited for)
+        const hipError_t err = st::run_clock_set(m.act, m.target, m.step, m.time, n, step0, *time, c->s);
         if (err != hipSuccess) return fail(c, -4, "march clock: %s", hipGetErrorString(err));
-        for (int it = 0; it < n; it++) {
-            int nb = 0;
-            Event e;
-            if (c->prof) prof_begin(c, KIND_RED * 3, e);
-            err = st::run_cfl_tstep(base_args(c), pc, hyper == 1 ? pt : nullptr, &nb, c->s);
-            if (err == hipSuccess)
-                err = st::run_dt(pc, pt, nb, 1, act, target, stepc, c->p.cfl_cal, hyper, first, run, dt, dt_last, hist,
-                                 step0, c->s);
-            if (c->prof) prof_end(c, e);
-            if (err != hipSuccess) return fail(c, -4, "march dt: %s", hipGetErrorString(err));
-            for (int loop = 0; loop < 2; loop++) {
-                const double *ra, *rb;
-                const int ns = rk_loop(c->p.rk_scheme, loop, &ra, &rb);
-                if (!ns) break;
-                for (int k = 0; k < ns; k++)                 // (QW: as stage_loop)
-                    TRY(seq_stage(c, a, ra[k], rb[k], 0.0, loop || k, last_stage(c->p.rk_scheme, loop, k), run));
-                err = st::run_clock(1, run, dt, tm, stepc, last_stage(c->p.rk_scheme, loop, ns - 1), c->s);
-                if (err != hipSuccess) return fail(c, -4, "march clock: %s", hipGetErrorString(err));
-            }
+        int rc = 0;
+        for (int it = 0; it < n && !rc; it++) {
+            if (it >= MARCH_AHEAD && !march_seen(c, it - MARCH_AHEAD + 1)) break;
+            rc = march_step(c, a, m, step0);
         }
+        // also after a launch that failed: the clock of the steps that ran
         HIPCHK(c, hipMemcpyAsync(c->m_clk_h, c->m_clk, sizeof(double) * (5 + n), hipMemcpyDeviceToHost, c->s));
         HIPCHK(c, hipStreamSynchronize(c->s));
         if (c->prof) prof_collect(c);
-        *time = c->m_clk_h[0];
-        *step = ((const int *)(c->m_clk_h + 3))[3];
-        const double *d = c->m_clk_h + 5;
-        for (int it = 0; it < *step - step0 && dt_out; it++) dt_out[done + it] = d[it];
+        const MarchClock h(c->m_clk_h);
+        *time = *h.time;
+        *step = *h.step;
+        for (int it = 0; it < *step - step0 && dt_out; it++) dt_out[done + it] = h.hist[it];
+        if (rc) return rc;
         if (*step - step0 < n)
-            return fail(c, -5, "non-finite or non-positive dt %g at step %d", d[*step - step0], *step);
+            return fail(c, -5, "non-finite or non-positive dt %g at step %d", h.hist[*step - step0], *step);
         done += n;
     }
     return 0;
@@ -1494,7 +1540,7 @@ int group_step(st_group *G)
         err = st::run_cfl_tstep(b, pc, m->p.hyper_param == 1 ? pt : nullptr, &nb, G->s);
         if (err == hipSuccess)
             err = st::run_dt(pc, pt, nb, m->ns, m->s_act, m->s_target, m->s_step, m->p.cfl_cal, m->p.hyper_param, 0,
-                             m->s_run, m->s_dt, m->s_dtlast, nullptr, 0, G->s);
+                             m->s_run, m->s_dt, m->s_dtlast, nullptr, 0, nullptr, G->s);
         if (err != hipSuccess) return st::set_call_error(-4, "group dt (%d points): %s", m->Mx, hipGetErrorString(err));
         b.act = m->s_run;
         b.sre = m->s_re;

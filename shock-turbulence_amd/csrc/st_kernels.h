@@ -148,9 +148,9 @@ hipError_t run_fill(double *p, long n, double v, hipStream_t s);
 hipError_t run_fill_slots(double *p, int nfields, long N, long ni, int nslot, const int *slots, const int *act,
                           double v, hipStream_t s);
 hipError_t run_fixp(const PassArgs &a, double *Qx, hipStream_t s);
-hipError_t run_dt(const double *pc, const double *pt, int nb, int nslot, const int *active, const int *target,
+hipError_t run_dt(const double *pc, const double *pt, int nb, int nslot, int *active, const int *target,
                   const int *stepc, double cfl_cal, int hyper, int first_step, int *run, double *dt, double *dt_last,
-                  double *hist, int hist0, hipStream_t s);
+                  double *hist, int hist0, int *seen, hipStream_t s);
 // the partials of both (pt null: of the CFL numbers alone)
 hipError_t run_cfl_tstep(const PassArgs &a, double *pc, double *pt, int *nblocks, hipStream_t s);
 hipError_t run_clock_set(int *active, int *target, int *stepc, double *time, int steps, int step, double t,

@@ -275,14 +275,16 @@ __global__ void __launch_bounds__(256) k_fixp(PassArgs a, double *Qx)
 // first_step = 1 applies them from the first step,
 // src/lddrk4_nonperiodic_sf.f:105).  stepc is the driver's step counter
 // (1 before the first step).  A slot runs this step (run = 1) while it is
-// active and its counter is below its target; with hist set, only if its dt is
-// positive and finite, and hist[step - hist0] records the dt.
+// active and its counter is below its target.  hist and seen (a single run's
+// march): hist[step - hist0] records the dt, and a slot whose dt is not positive
+// and finite does not run, now or later (active is cleared); seen, in host
+// memory, tells the host how many steps have their dt, -1 for such a slot.
 // The fold of up to 1024 partials a slot is a chain of dependent loads in one
 // thread (219 us at 64^3); 256 threads take four partials each (5 us).  A
 // maximum or minimum does not depend on the order, NaNs are passed over.
 __global__ void __launch_bounds__(256)
-k_dt(const double *pc, const double *pt, int nb, const int *active, const int *target, const int *stepc, double cfl_cal,
-     int hyper, int first_step, int *run, double *dt, double *dt_last, double *hist, int hist0)
+k_dt(const double *pc, const double *pt, int nb, int *active, const int *target, const int *stepc, double cfl_cal,
+     int hyper, int first_step, int *run, double *dt, double *dt_last, double *hist, int hist0, int *seen)
 {
     __shared__ double sh[4][4];
     const int slot = blockIdx.x;
@@ -324,8 +326,12 @@ k_dt(const double *pc, const double *pt, int nb, const int *active, const int *t
     }
     dt[slot] = t;
     dt_last[slot] = t;
-    if (hist) hist[step - hist0] = t;
-    run[slot] = !hist || (t > 0.0 && t < INFINITY);
+    run[slot] = 1;
+    if (!hist) return;
+    hist[step - hist0] = t;
+    const bool ok = t > 0.0 && t < INFINITY;
+    if (!ok) active[slot] = run[slot] = 0;
+    __hip_atomic_store(seen, ok ? step - hist0 + 1 : -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // time += dt after each RK loop; step += 1 after the second
@@ -544,12 +550,12 @@ hipError_t run_cfl_tstep(const PassArgs &a, double *pc, double *pt, int *nblocks
     return hipGetLastError();
 }
 
-hipError_t run_dt(const double *pc, const double *pt, int nb, int nslot, const int *active, const int *target,
+hipError_t run_dt(const double *pc, const double *pt, int nb, int nslot, int *active, const int *target,
                   const int *stepc, double cfl_cal, int hyper, int first_step, int *run, double *dt, double *dt_last,
-                  double *hist, int hist0, hipStream_t s)
+                  double *hist, int hist0, int *seen, hipStream_t s)
 {
     hipLaunchKernelGGL(k_dt, dim3((unsigned)nslot), dim3(256), 0, s, pc, pt, nb, active, target, stepc, cfl_cal, hyper,
-                       first_step, run, dt, dt_last, hist, hist0);
+                       first_step, run, dt, dt_last, hist, hist0, seen);
     return hipGetLastError();
 }
 

@@ -7,18 +7,15 @@
 #include <cstdio>
 #include <cstdlib>
 #include <array>
-#include <atomic>
 #include <chrono>
-#include <condition_variable>
 #include <cstring>
-#include <exception>
 #include <map>
-#include <mutex>
 #include <new>
 #include <thread>
 #include <vector>
 
 #include "../../include/st_api.h"
+#include "st_copiers.h"
 #include "st_internal.h"
 #include "st_kernels.h"
 
@@ -40,86 +37,6 @@ const char *kind_names[NKIND] = {
 struct Event {
     hipEvent_t a, b;
     int kind;             // pass kind * 3 + direction
-};
-
-// The helper threads of a context's host transfers, made at its first large
-// one and joined with it.  Between transfers they sleep; within one they share
-// each piece with the calling thread and poll for the next (a piece is some
-// tens of microseconds).  Threads that cannot be had are done without.
-class Copiers {
-public:
-    Copiers()
-    {
-        const int hw = (int)std::thread::hardware_concurrency();
-        const int n = hw - 1 < 0 ? 0 : hw - 1 < MOST ? hw - 1 : MOST;
-        try {
-            for (; have < n; have++) t[have] = std::thread([this, k = have] { work(k + 1); });
-        } catch (const std::exception &) {
-        }
-    }
-    ~Copiers()
-    {
-        set(&stop, true);
-        for (int k = 0; k < have; k++) t[k].join();
-    }
-    Copiers(const Copiers &) = delete;
-    Copiers &operator=(const Copiers &) = delete;
-    void begin() { set(&awake, true); }
-    void end() { set(&awake, false); }
-    // between begin() and end()
-    void copy(void *d, const void *s, size_t n)
-    {
-        dst = (char *)d;
-        src = (const char *)s;
-        size = n;
-        left.store(have, std::memory_order_relaxed);
-        turn.fetch_add(1, std::memory_order_release);
-        part(0);
-        while (left.load(std::memory_order_acquire) > 0) std::this_thread::yield();
-    }
-
-private:
-    static constexpr int MOST = 4;
-    void set(std::atomic<bool> *flag, bool v)
-    {
-        {
-            std::lock_guard<std::mutex> l(mu);
-            flag->store(v);
-        }
-        if (v) cv.notify_all();
-    }
-    void part(int k) const
-    {
-        const size_t each = (size / (have + 1) + 63) & ~(size_t)63, o = each * k;
-        if (o < size) std::memcpy(dst + o, src + o, size - o < each || k == have ? size - o : each);
-    }
-    void work(int k)
-    {
-        for (long seen = 0;;) {
-            if (turn.load(std::memory_order_acquire) != seen) {
-                seen++;
-                part(k);
-                left.fetch_sub(1, std::memory_order_release);
-            } else if (stop) {
-                return;
-            } else if (awake) {
-                std::this_thread::yield();
-            } else {
-                std::unique_lock<std::mutex> l(mu);
-                cv.wait(l, [this] { return stop || awake; });
-            }
-        }
-    }
-    std::thread t[MOST];
-    int have = 0;
-    char *dst = nullptr;
-    const char *src = nullptr;
-    size_t size = 0;
-    std::mutex mu;
-    std::condition_variable cv;
-    std::atomic<bool> stop{false}, awake{false};
-    std::atomic<long> turn{0};
-    std::atomic<int> left{0};
 };
 
 // The clock block of st_march: time, dt, the last dt, four integers, then the
@@ -170,7 +87,7 @@ struct st_ctx {
     std::vector<int> act_h;
     int nact = 0;                   // active slots, listed in s_list (launch grids cover these only)
     std::vector<hipGraphExec_t> graphs;   // one batch step, captured per active-slot count
-    Copiers *crew = nullptr;                    // threads of the large host transfers
+    st::Copiers *crew = nullptr;                // threads of the large host transfers
     void *stage[2] = {nullptr, nullptr};        // pinned transfer buffers, made at the first large transfer
     hipEvent_t stage_ev[2] = {nullptr, nullptr};
     double *m_clk = nullptr;        // clock and dts of st_march (MarchClock, device), and its pinned host copy
@@ -706,16 +623,9 @@ bool stage_ready(st_ctx *c)
             return false;
         }
     }
-    if (!c->crew) c->crew = new (std::nothrow) Copiers;
+    if (!c->crew) c->crew = new (std::nothrow) st::Copiers;
     return c->crew != nullptr;
 }
-
-// The threads awake for one transfer.
-struct Awake {
-    Copiers &crew;
-    explicit Awake(Copiers &c) : crew(c) { crew.begin(); }
-    ~Awake() { crew.end(); }
-};
 
 // The i-th piece of a transfer of nfields fields of w bytes, at most
 // STAGE_BYTES: several whole fields (rows > 1 device rows), or part of one.
@@ -750,7 +660,6 @@ int up(st_ctx *c, double *dev, const double *host, long nfields, int slot = 0)
         return 0;
     }
     const long n = pieces_of(w, nfields);
-    const Awake on(*c->crew);
     for (long i = 0; i < n; i++) {
         const Piece p = piece(w, nfields, i);
         const int k = (int)(i & 1);
@@ -772,7 +681,7 @@ int down(st_ctx *c, double *host, const double *dev, long nfields, int slot = 0)
         HIPCHK(c, hipStreamSynchronize(c->s));
     } else {
         const long n = pieces_of(w, nfields);
-        const Awake on(*c->crew);
+        c->crew->wake();                                      // while the first piece comes
         for (long i = 0; i <= n; i++) {
             if (i < n) {                                      // the next piece comes while the last is copied out
                 const Piece p = piece(w, nfields, i);

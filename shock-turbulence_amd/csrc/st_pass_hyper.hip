@@ -305,8 +305,16 @@ struct PassGaussHdiv {
 };
 
 
+// The fluxes are stored for x and y alone, and the pass that forms them takes
+// the z derivative.
+static bool flux_dir(int kind, int dir)
+{
+    return kind == K_HDIV ? dir != 2 : kind == K_GAUSS_ETA_LAST ? dir == 2 : true;
+}
+
 hipError_t launch_hyper(int kind, const DirTab &t, int nt, int dir, int My, int Mz, int Mx, const PassArgs &a, hipStream_t s)
 {
+    if (!flux_dir(kind, dir)) return hipErrorInvalidValue;
     switch (kind) {
     case K_LAP2: return launch<PassLap2>(t, nt, dir, My, Mz, Mx, a, s);
     case K_LAP2_LAST: return launch<PassLap2Gauss, false>(t, nt, dir, My, Mz, Mx, a, s);
@@ -320,6 +328,7 @@ hipError_t launch_hyper(int kind, const DirTab &t, int nt, int dir, int My, int 
 
 hipError_t launch_hyper_ragged(int kind, const RaggedSpec &sp, hipStream_t s)
 {
+    if (!flux_dir(kind, sp.dir)) return hipErrorInvalidValue;
     switch (kind) {
     case K_LAP2: return launch_ragged<PassLap2>(sp, s);
     case K_LAP2_LAST: return launch_ragged<PassLap2Gauss>(sp, s);

@@ -475,10 +475,14 @@ DEV double scan_in(double e, CTab &T, int c)
 // 1+rho^2 or 1/kappa already folded in) and returns x.
 // Order 1 (OP 0, 1): x = (1 - rho S^-1)^-1 (1 - rho S)^-1 r,
 // order 2: x = (1 - a1 S^-1 - a2 S^-2)^-1 (1 - a1 S - a2 S^2)^-1 r.
-template <int OP, int M, int P, bool NP, bool AL>
+// FULL: the scan over the whole line also where the in-row one would do (the
+// operators that a host program calls by themselves: every point keeps its
+// digits however small it is beside the line's largest, and one that is not
+// finite reaches the whole line).
+template <int OP, int M, bool FULL = false, int P, bool NP, bool AL>
 DEV void solve(double (&r)[M], CTab &T, const Lane<M, P, NP, AL> &L)
 {
-    constexpr int K = OP == 2 ? 2 : 1, STEPS = scan_steps<OP>(M, P);
+    constexpr int K = OP == 2 ? 2 : 1, STEPS = FULL ? 0 : scan_steps<OP>(M, P);
     const double a1 = T.a1, a2 = T.a2;
     const int c = L.c;
     // forward recurrence inside the chunk (zero incoming state)
@@ -562,7 +566,7 @@ DEV double line_value(const double (&x)[M], const Lane<M, P, NP, AL> &L, int row
 
 // Boundary correction x -= Z q, q = G yb (the np_* tables of OpTab; Z
 // itself is applied through the recurrences, below).
-template <int OP, int M, int P, bool NP, bool AL>
+template <int OP, bool FULL = false, int M, int P, bool NP, bool AL>
 DEV void np_fix(double (&x)[M], CTab &T, const Lane<M, P, NP, AL> &L)
 {
     constexpr int n = M * P, MB = OP == 2 ? 6 : 4;
@@ -598,7 +602,7 @@ DEV void np_fix(double (&x)[M], CTab &T, const Lane<M, P, NP, AL> &L)
         }
         z[k] = v;
     }
-    solve<OP, M>(z, T, L);
+    solve<OP, M, FULL>(z, T, L);
 #pragma unroll
     for (int k = 0; k < M; k++) x[k] -= z[k];
 }
@@ -747,7 +751,7 @@ DEV void closure_rows(const double (&w)[W], double K, const Lane<M, P, NP, AL> &
 
 // First derivative: K.k = cadd*sx(1)*(N-1)*(1+rho^2), K.a, K.b its products
 // with the stencil's weights on +-1 and +-2.
-template <int M, int W, int P, bool NP, bool AL>
+template <int M, bool FULL = false, int W, int P, bool NP, bool AL>
 DEV void op_d1(const double (&w)[W], const Scale1 &K, CTab &T, const Lane<M, P, NP, AL> &L, double (&out)[M])
 {
     constexpr int H = (W - M) / 2;
@@ -757,15 +761,15 @@ DEV void op_d1(const double (&w)[W], const Scale1 &K, CTab &T, const Lane<M, P, 
         out[k] = fma(K.a, w[i + 1] - w[i - 1], K.b * (w[i + 2] - w[i - 2]));
     }
     if constexpr (NP) closure_rows<0, M>(w, K.k, L, out);
-    solve<0, M>(out, T, L);
-    if constexpr (NP && M * P >= 64) np_fix_ends<0>(out, T, L);
-    else if constexpr (NP) np_fix<0>(out, T, L);
+    solve<0, M, FULL>(out, T, L);
+    if constexpr (NP && M * P >= 64 && !FULL) np_fix_ends<0>(out, T, L);
+    else if constexpr (NP) np_fix<0, FULL>(out, T, L);
 }
 
 // Second derivative: K.k = (N-1)^2*sx(2)*(1+rho^2), K.a, K.b, K.c its products
 // with the weights on +-1, +-2 and (the coefficients as shipped only,
 // 0 otherwise) +-3, K.d with the centre weight.
-template <int M, int W, int P, bool NP, bool AL>
+template <int M, bool FULL = false, int W, int P, bool NP, bool AL>
 DEV void op_d2(const double (&w)[W], const Scale2 &K, CTab &T, const Lane<M, P, NP, AL> &L, double (&out)[M])
 {
     constexpr int H = (W - M) / 2;
@@ -783,9 +787,9 @@ DEV void op_d2(const double (&w)[W], const Scale2 &K, CTab &T, const Lane<M, P, 
         for (int k = 0; k < M; k++) out[k] = fma(K.c, x[k + HALO + 3] + x[k + HALO - 3], out[k]);
     }
     if constexpr (NP) closure_rows<1, M>(w, K.k, L, out);
-    solve<1, M>(out, T, L);
-    if constexpr (NP && M * P >= 64) np_fix_ends<1>(out, T, L);
-    else if constexpr (NP) np_fix<1>(out, T, L);
+    solve<1, M, FULL>(out, T, L);
+    if constexpr (NP && M * P >= 64 && !FULL) np_fix_ends<1>(out, T, L);
+    else if constexpr (NP) np_fix<1, FULL>(out, T, L);
 }
 
 // Eighth-order compact filter: K = 1/kappa.

@@ -18,7 +18,7 @@ struct PassD1 : NoReuse {
 #pragma unroll
         for (int k = 0; k < M; k++) f[k] = L.ld(0, k);
         window<M>(f, L, w);
-        op_d1<M>(w, a.K1, a.tab()->op[0], L, out[0]);
+        op_d1<M, true>(w, a.K1, a.tab()->op[0], L, out[0]);
     }
     template <class A>
     DEV static void store(const Geo &, const A &a, long gi, const double *v)
@@ -38,10 +38,10 @@ struct PassD2 : NoReuse {
 #pragma unroll
         for (int k = 0; k < M; k++) f[k] = L.ld(0, k);
         window<M>(f, L, w);
-        op_d2<M>(w, a.K2, a.tab()->op[1], L, d2);
+        op_d2<M, true>(w, a.K2, a.tab()->op[1], L, d2);
 #pragma unroll
         for (int k = 0; k < M; k++) L.st(1, k, d2[k]);
-        if (a.iadd) op_d1<M>(w, a.K1, a.tab()->op[0], L, out[0]);
+        if (a.iadd) op_d1<M, true>(w, a.K1, a.tab()->op[0], L, out[0]);
         else {
 #pragma unroll
             for (int k = 0; k < M; k++) out[0][k] = 0.0;

@@ -1235,7 +1235,7 @@ int march_step(st_ctx *c, const st::PassArgs &a, const MarchClock &m, int step0)
 }
 
 // Wait until the device has decided on `steps` steps of a chunk; false once
-// it has refused one (or the stream has stopped on an error).
+// it has refused one, or the stream has stopped or cannot be asked.
 bool march_seen(st_ctx *c, int steps)
 {
     for (;;) {
@@ -1285,6 +1285,7 @@ extern "C" int st_march(st_ctx *c, int nsteps, double *time, int *step, double *
         *step = *h.step;
         for (int it = 0; it < *step - step0 && dt_out; it++) dt_out[done + it] = h.hist[it];
         if (rc) return rc;
+        if (*step - step0 < n && *h.act) return fail(c, -3, "march stopped at step %d", *step);
         if (*step - step0 < n)
             return fail(c, -5, "non-finite or non-positive dt %g at step %d", h.hist[*step - step0], *step);
         done += n;

@@ -606,10 +606,18 @@ bool last_stage(int scheme, int loop, int k)
 // Host arrays hold one instance (nfields x ni, contiguous); on the device
 // the fields of slot `slot` sit at dev + f*N + slot*ni.
 // Transfers of 1 MiB and more of pageable arrays go through two pinned buffers
-// of the context, filled or emptied by several threads while the other is on the bus.  (The
-// runtime's own path for pageable memory copies, and takes the page faults of
-// a new array, on one thread.  19.7 MB up 558 -> 517 us, down 1068 -> 509, down
-// into a new array 1389 -> 880.)
+// of the context, filled or emptied by several threads while the other is on
+// the bus.  (The runtime's own path for pageable memory copies, and takes the
+// page faults of a new array, on one thread.)  us of one transfer by itself,
+// runtime / staged, of an array used before and of a new one:
+//              1.3 MB     4.4 MB     10.5 MB    20.5 MB     41.3 MB      83.9 MB
+//   up         513/75     148/161    317/301    588/563     1465/1073    2988/2130
+//   up, new    82/76      147/175    319/313    692/591     1482/1245    3119/2286
+//   down       102/75     236/148    647/295    1220/541    2421/1050    5005/2103
+//   down, new  101/76     232/151    620/310    1209/552    4112/2343    8396/4527
+// Between 2 and 6 MB a bare upload of a new array loses up to 28 us; within the
+// calls that upload, none does (a slot loaded, runtime / staged: 4.4 MB 287/282,
+// 7.0 MB 451/405, 10.5 MB 534/443).
 constexpr size_t STAGE_BYTES = 2 << 20, STAGE_MIN = 1 << 20;
 
 // The buffers, at the first such transfer; without them the runtime's path

@@ -58,7 +58,7 @@ public:
 
 private:
     static constexpr int MOST = 4;
-    static constexpr std::chrono::microseconds SPIN{200};
+    static constexpr std::chrono::microseconds SPIN{100};
     // wake what sleeps.  A thread counts itself asleep before it looks at turn,
     // calls and stop for the last time, and the caller changes these before it
     // reads the count, so one of the two sees the other.

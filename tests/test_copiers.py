@@ -33,7 +33,7 @@ int main()
     for (auto &x : a) x = (unsigned char)((r = r * 1664525u + 1013904223u) >> 24);
     st::Copiers c;
     const size_t sizes[] = {0, 1, 63, 64, 65, 319, 320, 321, 4095, 65536, (1 << 20) + 1, 2 << 20, most};
-    for (int pause : {0, 20, 190, 200, 210, 1000})
+    for (int pause : {0, 20, 90, 100, 110, 1000})
         for (int k = 0; k < 30; k++)
             for (size_t n : sizes) {
                 std::memset(b.data(), 0, n + 2);
@@ -59,5 +59,5 @@ def test_copies_and_idle_time(tmp_path):
     subprocess.run(["g++", "-std=c++17", "-O2", "-Wall", "-pthread", str(src), "-o", str(exe)], check=True)
     r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=100)
     assert r.returncode == 0, r.returncode
-    # up to four threads polling for half a second would take 2 s; 200 us each are allowed
+    # up to four threads polling for half a second would take 2 s; 100 us each are allowed
     assert float(r.stdout) < 0.1, r.stdout

@@ -869,7 +869,7 @@ int kerr(st_ctx *c, hipError_t e, const char *what)
 // /GRAD/ still zero).  The passes are those of a stage, on fields of their own:
 // the 19 of T5, tB, tC, dQp and L2ep, which follow each other and which a stage
 // rewrites before reading (what st_rhs leaves for st_hyper_rhs stays as it is).
-// 17 launches (35 as single operators and sums).
+// 18 launches (35 as single operators and sums); 14 without the sensor.
 int seq_compute_hyper(st_ctx *c, int slot, int use_grad)
 {
     const long off = (long)slot * c->ni, N = c->N, ni = c->ni;

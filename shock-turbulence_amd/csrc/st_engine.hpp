@@ -74,7 +74,7 @@ DEV long tile_of(const Geo &g, long wg)
 // values spill).  The compute phase and the staging of x and z tiles of 16
 // or more lines stay free of bank conflicts; the staging of y tiles and of
 // narrower x and z tiles takes up to M-way conflicts.  Each pass names the
-// layout that measured faster for it (LDS_ADD).
+// layout that measured faster for it (lds_add).
 template <int M>
 HD int lds_g(int b, int B)
 {

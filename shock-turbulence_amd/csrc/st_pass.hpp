@@ -148,7 +148,8 @@ struct mf_n<T, std::void_t<decltype(T::NMF)>> { static constexpr int value = T::
 // Gaussian 0.27 -> 0.19); a strided pass gains only with tiles of 16 lines or
 // more, whose rows are whole 128-byte lines (narrower rows share a line
 // between tiles: the x gradient pass on 8-line tiles 0.58 -> 0.69 ms).  The
-// filters and the z gradient pass, on narrow tiles, name none.
+// filters and the plain z gradient pass, on narrow tiles, name none; the
+// two-round z gradient pass does, for its 16-line tiles of 512 threads.
 template <class T, class = void>
 struct stream_n { static constexpr int value = 0; };
 template <class T>

@@ -43,11 +43,13 @@ namespace st {
 // each times (1/3 + bulk) mu into the momentum component it belongs to and,
 // times that velocity, into the energy.  The x sweep runs first, so the z
 // and y sweeps find the derivatives they need.
-// TWO (the z sweep at 8 points per lane): the two mixed inputs are staged in
+// TWO (the z sweep, two rounds of staging): the two mixed inputs are staged in
 // the slots of v and rho, whose values wait in registers (NHOLD) until the
-// mixed terms are done (compute_a); five slots instead of seven, so that
-// 8-line tiles fit two workgroups per CU (0.70 -> 0.645 ms at 256^3; at 4
-// points per lane the extra phase costs more than it gives, 0.70 -> 0.79).
+// mixed terms are done (compute_a); five slots instead of seven.  At 8 points
+// per lane 8-line tiles of 256 threads then fit two workgroups per CU (0.70 ->
+// 0.645 ms at 256^3); at 4 to 7, 16-line tiles of 512 threads, which stream (128^3
+// stage 710 -> 699 us), while on 256 threads the extra phase costs more than it
+// gives (256^3 at 4 points per lane 0.70 -> 0.79 ms).
 template <int DIR, int MW, bool TWO_ = false>
 struct PassGrad {
     static constexpr bool TWO = TWO_, CROSS = DIR == 1;

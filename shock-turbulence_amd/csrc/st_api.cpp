@@ -42,6 +42,7 @@ struct Event {
 // The clock block of st_march: time, dt, the last dt, four integers, then the
 // dt of each step of a chunk.
 struct MarchClock {
+    static constexpr int SIZE = 5 + MARCH_CHUNK;
     double *time, *dt, *dt_last;
     int *act, *run, *target, *step;
     double *hist;
@@ -77,9 +78,9 @@ struct st_ctx {
     double *buf = nullptr;
     double *Q, *QW, *dQ, *G, *L2e, *S, *Cb, *L2S, *L4e, *L4S, *eta, *Hc, *T5, *tB, *tC;
     double *dQp, *L2ep;             // z and x partials of the first-derivative passes
-    double *red = nullptr;          // reduction partials (device)
-    double *red_h = nullptr;        // pinned host copy
-    long red_n = 0;                 // doubles in red / red_h
+    double *red = nullptr;          // reduction partials (device), then the clock of st_march
+    double *red_h = nullptr;        // pinned host copy of both, then m_seen
+    long red_n = 0;                 // doubles of the partials
     // per-slot state of a batch (device): active flag, run flag of the
     // current step, step target, driver step counter, 1/Re, dt, time
     int *s_act = nullptr, *s_run, *s_target, *s_step, *s_list;
@@ -90,9 +91,9 @@ struct st_ctx {
     st::Copiers *crew = nullptr;                // threads of the large host transfers
     void *stage[2] = {nullptr, nullptr};        // pinned transfer buffers, made at the first large transfer
     hipEvent_t stage_ev[2] = {nullptr, nullptr};
-    double *m_clk = nullptr;        // clock and dts of st_march (MarchClock, device), and its pinned host copy
+    double *m_clk = nullptr;        // clock and dts of st_march (MarchClock), and its host copy
     double *m_clk_h = nullptr;
-    int *m_seen = nullptr;          // pinned, written by the device: steps of the chunk with a dt, -1 once one was refused
+    int *m_seen = nullptr;          // written by the device: steps of the chunk with a dt, -1 once one was refused
     double *spg = nullptr;          // sponge: sigma per x index, then the left and right reference states
     int spg_left = 0;               // x indices [0, spg_left) take the left reference state
     int use_graph = 1;
@@ -444,16 +445,16 @@ extern "C" int st_batch_create(const st_grid *grid, const st_params *params, int
     const size_t ns = (size_t)nslots;
     if ((e = hipMalloc(&c->buf, sizeof(double) * nf * c->N)) != hipSuccess ||
         (e = hipMalloc(&c->td, sizeof(st::DirTab) * 6)) != hipSuccess ||
-        (e = hipMalloc(&c->red, sizeof(double) * c->red_n)) != hipSuccess ||
-        (e = hipHostMalloc(&c->red_h, sizeof(double) * c->red_n)) != hipSuccess ||
-        (e = hipMalloc(&c->m_clk, sizeof(double) * (5 + MARCH_CHUNK))) != hipSuccess ||
-        (e = hipHostMalloc(&c->m_clk_h, sizeof(double) * (5 + MARCH_CHUNK))) != hipSuccess ||
-        (e = hipHostMalloc(&c->m_seen, sizeof(int), hipHostMallocCoherent)) != hipSuccess ||
+        (e = hipMalloc(&c->red, sizeof(double) * (c->red_n + MarchClock::SIZE))) != hipSuccess ||
+        (e = hipHostMalloc(&c->red_h, sizeof(double) * (c->red_n + MarchClock::SIZE + 1), hipHostMallocCoherent)) != hipSuccess ||
         (e = hipMalloc(&sp, ns * (6 * sizeof(int) + 4 * sizeof(double)))) != hipSuccess) {
         fail(c, -3, "device allocation: %s", hipGetErrorString(e));
         *out = c;
         return -3;
     }
+    c->m_clk = c->red + c->red_n;
+    c->m_clk_h = c->red_h + c->red_n;
+    c->m_seen = (int *)(c->m_clk_h + MarchClock::SIZE);
     c->s_re = (double *)sp;
     c->s_dt = c->s_re + ns;
     c->s_time = c->s_dt + ns;
@@ -521,9 +522,6 @@ extern "C" void st_ctx_destroy(st_ctx *c)
         if (c->stage[k]) (void)hipHostFree(c->stage[k]);
         if (c->stage_ev[k]) (void)hipEventDestroy(c->stage_ev[k]);
     }
-    if (c->m_clk) (void)hipFree(c->m_clk);
-    if (c->m_clk_h) (void)hipHostFree(c->m_clk_h);
-    if (c->m_seen) (void)hipHostFree(c->m_seen);
     if (c->s) (void)hipStreamDestroy(c->s);
     delete c;
 }

@@ -246,7 +246,7 @@ void set_tab(const st_ctx *c, st::PassArgs &a, int lay, int dir, double cadd)
     const double k1 = cadd * c->sx1[dir] * (double)(t.n - 1) * t.op[0].scale;   // fac of src/derivCDopt6_periodic.f:181
     const double k2 = t.s2 * t.op[1].scale;
     a.K1 = {k1, k1 * C.a1, k1 * C.b1};
-    a.K2 = {k2, k2 * C.a2, k2 * C.b2, k2 * C.c2, k2 * C.d2};
+    a.K2 = {k2, k2 * (C.a2 + 2.0 * C.b2), k2 * C.b2, k2 * C.c2, k2 * (2.0 * (C.a2 + C.b2) - C.d2)};
 }
 
 int pass(st_ctx *c, int kind, int dir, st::PassArgs a, double cadd = 1.0)

@@ -766,25 +766,30 @@ DEV void op_d1(const double (&w)[W], const Scale1 &K, CTab &T, const Lane<M, P, 
     else if constexpr (NP) np_fix<0, FULL>(out, T, L);
 }
 
-// Second derivative: K.k = (N-1)^2*sx(2)*(1+rho^2), K.a, K.b, K.c its products
-// with the weights on +-1, +-2 and (the coefficients as shipped only,
-// 0 otherwise) +-3, K.d with the centre weight.
+// Second derivative: K.k = (N-1)^2*sx(2)*(1+rho^2).  The stencil is taken on
+// second differences: with a (+-1) and b (+-2) the weights, a (w1 - 2 w0 + w-1) +
+// b (w2 - 2 w0 + w-2) = (a + 2b) s0 + b (s1 + s-1), as many operations as on the
+// values.  A constant then gives 0 whatever the weights' rounding, and what is
+// rounded is of the size of the differences (weights scaled one by one on the
+// values: up to 3.6 roundings of a constant).  K.e and K.b are the scaled weights;
+// K.c (+-3) and K.z (what the centre weight then lacks) are 0 but for the
+// coefficients as shipped.
 template <int M, bool FULL = false, int W, int P, bool NP, bool AL>
 DEV void op_d2(const double (&w)[W], const Scale2 &K, CTab &T, const Lane<M, P, NP, AL> &L, double (&out)[M])
 {
     constexpr int H = (W - M) / 2;
+    double s[M + 2];                       // second differences of points -1..M
 #pragma unroll
-    for (int k = 0; k < M; k++) {
-        const int i = k + H;
-        out[k] = fma(K.a, w[i + 1] + w[i - 1], fma(K.b, w[i + 2] + w[i - 2], -K.d * w[i]));
-    }
+    for (int j = 0; j < M + 2; j++) s[j] = (w[H + j] - w[H + j - 1]) - (w[H + j - 1] - w[H + j - 2]);
+#pragma unroll
+    for (int k = 0; k < M; k++) out[k] = fma(K.e, s[k + 1], K.b * (s[k] + s[k + 2]));
     if (K.c != 0.0) {                      // the same on every lane
         double v[M], x[M + 2 * HALO];
 #pragma unroll
         for (int k = 0; k < M; k++) v[k] = w[k + H];
         window<M>(v, L, x);
 #pragma unroll
-        for (int k = 0; k < M; k++) out[k] = fma(K.c, x[k + HALO + 3] + x[k + HALO - 3], out[k]);
+        for (int k = 0; k < M; k++) out[k] = fma(K.c, x[k + HALO + 3] + x[k + HALO - 3], fma(K.z, v[k], out[k]));
     }
     if constexpr (NP) closure_rows<1, M>(w, K.k, L, out);
     solve<1, M, FULL>(out, T, L);

@@ -66,7 +66,7 @@ struct Scale1 {
     double k, a, b;               // +-1, +-2
 };
 struct Scale2 {
-    double k, a, b, c, d;         // +-1, +-2, +-3, centre
+    double k, e, b, c, z;         // second differences, those beside, +-3, value (op_d2)
 };
 
 // Physical parameters used in kernels.
